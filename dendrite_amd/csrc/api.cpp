@@ -140,6 +140,8 @@ struct dh_plan {
     bool prefill;
     uint32_t* row_len;
     dh::ItemLim* item_lim;
+    uint32_t* split_rows;    // queries of a split tail's blocks, n_split_rows of them
+    uint32_t n_split_rows;
     dh_plan_stats stats;
     size_t ws_bytes;
     size_t ws_lse_off;
@@ -147,9 +149,10 @@ struct dh_plan {
     // for dh_plan_update, and where items and pages start in dev (words).
     std::vector<uint32_t> tail_off, tail_n, tail_cap, tail_item_ptr, tail_items;
     size_t items_word, pages_word;
-    // Prefill plans with one partial state per row, and direct decode plans
-    // (each workgroup merges its own rows): the attention kernel writes out
-    // and there is no merge launch.
+    // Prefill plans with one partial state per row (split tails aside, whose
+    // rows a small merge writes), and direct decode plans (each workgroup
+    // merges its own rows): the attention kernel writes out and there is no
+    // merge launch.
     bool direct;
     uint32_t max_slots;      // most partial states of one sequence
     uint32_t uniform_slots;  // every sequence's count of partial states when they are all equal, else 0
@@ -610,7 +613,8 @@ static dh_status upload_plan(dh_backend* be, const dh_attn_config* cfg, const dh
     const size_t o_sp = align_up(o_ss + hp.seqslots.size() * sizeof(dh::SeqSlot), 256);
     const size_t o_rl = align_up(o_sp + hp.slot_ptr.size() * sizeof(uint32_t), 256);
     const size_t o_il = align_up(o_rl + hp.row_len.size() * sizeof(uint32_t), 256);
-    const size_t total = align_up(o_il + hp.item_lim.size() * sizeof(dh::ItemLim), 256);
+    const size_t o_sr = align_up(o_il + hp.item_lim.size() * sizeof(dh::ItemLim), 256);
+    const size_t total = align_up(o_sr + hp.split_rows.size() * sizeof(uint32_t), 256);
     std::vector<uint8_t> blob(total, 0);
     memcpy(blob.data() + o_items, hp.items.data(), hp.items.size() * sizeof(dh::Item));
     memcpy(blob.data() + o_pages, hp.pages.data(), hp.pages.size() * sizeof(uint32_t));
@@ -619,6 +623,8 @@ static dh_status upload_plan(dh_backend* be, const dh_attn_config* cfg, const dh
     if (!hp.row_len.empty()) memcpy(blob.data() + o_rl, hp.row_len.data(), hp.row_len.size() * sizeof(uint32_t));
     if (!hp.item_lim.empty())
         memcpy(blob.data() + o_il, hp.item_lim.data(), hp.item_lim.size() * sizeof(dh::ItemLim));
+    if (!hp.split_rows.empty())
+        memcpy(blob.data() + o_sr, hp.split_rows.data(), hp.split_rows.size() * sizeof(uint32_t));
     dh::DeviceGuard guard(be->device);
     hipError_t e = guard.error();
     if (e == hipSuccess) e = hipMalloc(&pl->dev, total);
@@ -635,9 +641,12 @@ static dh_status upload_plan(dh_backend* be, const dh_attn_config* cfg, const dh
     pl->slot_ptr = reinterpret_cast<uint32_t*>(pl->dev + o_sp);
     pl->row_len = prefill ? reinterpret_cast<uint32_t*>(pl->dev + o_rl) : nullptr;
     pl->item_lim = prefill ? reinterpret_cast<dh::ItemLim*>(pl->dev + o_il) : nullptr;
+    pl->split_rows = prefill ? reinterpret_cast<uint32_t*>(pl->dev + o_sr) : nullptr;
+    pl->n_split_rows = uint32_t(hp.split_rows.size());
     const size_t rows = size_t(hp.num_slots) * cfg->num_heads;
-    // Partial O: fp32 for f32 q, else f16 scaled per row (dh::PartialLse).
-    const size_t o_bytes = cfg->q_dtype == DH_DTYPE_F32 ? sizeof(float) : sizeof(uint16_t);
+    // Partial O: fp32 for f32 q and split prefill tails, else f16 scaled per
+    // row (dh::PartialLse).
+    const size_t o_bytes = cfg->q_dtype == DH_DTYPE_F32 || hp.split_tail ? sizeof(float) : sizeof(uint16_t);
     pl->ws_lse_off = align_up(rows * cfg->head_dim * o_bytes, 256);
     pl->ws_bytes = align_up(pl->ws_lse_off + rows * sizeof(dh::PartialLse), 256);
     fill_stats(hp, batch, &pl->stats);
@@ -655,7 +664,7 @@ static dh_status upload_plan(dh_backend* be, const dh_attn_config* cfg, const dh
     for (uint32_t v = 0; v < batch; ++v)
         if (hp.slot_ptr[v + 1] - hp.slot_ptr[v] != pl->max_slots) pl->uniform_slots = 0;
     for (uint32_t v = 0; prefill && v < batch; ++v)
-        if (hp.slot_ptr[v + 1] - hp.slot_ptr[v] != 1) pl->direct = false;
+        if (!hp.split_tail && hp.slot_ptr[v + 1] - hp.slot_ptr[v] != 1) pl->direct = false;
     pl->items_word = o_items / sizeof(uint32_t);
     pl->pages_word = o_pages / sizeof(uint32_t);
     retain(be);
@@ -751,6 +760,8 @@ dh_status dh_plan_create_prefill(dh_backend* be, const dh_attn_config* cfg, cons
     in.group_rows = uint32_t(dh::group_rows(false, int(cfg->head_dim)));
     in.causal = causal != 0;
     in.chunk_pages = chunk_pages;
+    // Workgroups per CU by the kernel's LDS: 40 KiB, 72 KiB or more than 80.
+    in.wg_slots = 256u * (cfg->head_dim == 64 ? 4u : cfg->head_dim == 128 ? 2u : 1u);
     dh::HostPlan hp;
     std::string err;
     const int rc = dh::build_prefill_plan(in, hp, err);
@@ -972,6 +983,17 @@ static dh_status decode_impl(dh_backend* be, const dh_pool* pool, const dh_plan*
         hipError_t e = hipError_t(dh::launch_attend(a, pl->n_tasks, c.q_dtype, c.kv_format, c.head_dim,
                                                     pl->prefill, stream));
         if (e != hipSuccess) return fail(DH_EHIP, "attention launch failed: %s", hipGetErrorString(e));
+    }
+    if ((mask & 2u) && pl->n_split_rows) {
+        dh::MergeArgs m{};
+        m.slot_ptr = pl->slot_ptr;
+        m.ws_o = ws_o;
+        m.ws_lse = ws_lse;
+        m.out = out;
+        m.hq = c.num_heads;
+        const hipError_t e = hipError_t(dh::launch_prefill_merge(m, pl->split_rows, pl->n_split_rows, c.q_dtype,
+                                                                 c.head_dim, stream));
+        if (e != hipSuccess) return fail(DH_EHIP, "merge launch failed: %s", hipGetErrorString(e));
     }
     if ((mask & 2u) && !pl->direct) {
         dh::MergeArgs m{};

@@ -1632,6 +1632,15 @@ __device__ __forceinline__ void write_partial_dma(const AttendArgs& a, const Ite
         const uint32_t row = uint32_t(rt * kWaves + wave) * kTileRows + c;
         const float lt = L[rt][0];
         const float inv = lt > 0.f ? 1.f / lt : 0.f;
+        if (PF && a.out_direct && (it.flags & kItemSplit)) {   // one of the row's chunks, in f32
+            if (row < it.nrows) {
+                float* o = static_cast<float*>(a.ws_o) + uint64_t(dst[rt]) * D;
+                #pragma unroll
+                for (int e = 0; e < EPL; ++e) *reinterpret_cast<f4*>(o + 16 * e + 4 * g) = O[rt][e] * inv;
+                if (g == 0) a.ws_lse[dst[rt]] = PartialLse{lt > 0.f ? m[rt] + log2f(lt) : kNegInf, 0.f};
+            }
+            continue;
+        }
         if (PF && a.out_direct) {   // the row's only partial state is its output
             if (row < it.nrows) {
                 uint8_t* o = static_cast<uint8_t*>(a.out_direct) + rtg.qoff[rt];
@@ -2584,6 +2593,47 @@ __global__ __launch_bounds__(256) void merge_kernel(MergeArgs a) {
     const uint32_t n = a.uniform_slots ? a.uniform_slots
                                        : ((a.seq_bad && a.seq_bad[b]) ? 0u : a.slot_ptr[b + 1] - s0);
     merge_row<D, OUT, NV>(a.ws_o, a.ws_lse, a.out, a.hq, b, qh, s0, n, lane);
+}
+
+// Rows of a prefill plan's split blocks: one wave per (row, query head).
+// Launch-bound (a few hundred rows of 2-12 states); the states are read one
+// after another, their loads independent of the running sums, so several
+// are in flight.  f32 states, so a split row holds no less than a whole one
+// (error against 64 bits 0.0034 either way on the case at prefill_tail).
+template <int D, bool F16>
+__global__ __launch_bounds__(256) void prefill_merge_kernel(MergeArgs a, const uint32_t* rows, uint32_t n) {
+    constexpr int PL = D / 64;
+    const int lane = threadIdx.x & 63;
+    const uint32_t w = blockIdx.x * kWaves + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    if (w >= n * a.hq) return;
+    const uint32_t i = w / a.hq, qh = w - i * a.hq;
+    const uint32_t v = __builtin_amdgcn_readfirstlane(rows[i]);
+    const uint32_t s0 = __builtin_amdgcn_readfirstlane(a.slot_ptr[v]);
+    const uint32_t s1 = __builtin_amdgcn_readfirstlane(a.slot_ptr[v + 1]);
+    float M = kNegInf;
+    for (uint32_t s = s0; s < s1; ++s) M = fmaxf(M, a.ws_lse[uint64_t(s) * a.hq + qh].lse);
+    float acc[PL], W = 0.f;
+    #pragma unroll
+    for (int k = 0; k < PL; ++k) acc[k] = 0.f;
+    if (M != kNegInf) {
+        #pragma unroll 4
+        for (uint32_t s = s0; s < s1; ++s) {
+            const uint64_t row = uint64_t(s) * a.hq + qh;
+            const float l = a.ws_lse[row].lse;
+            const float wk = l == kNegInf ? 0.f : fast_exp2(l - M);
+            const float* o = static_cast<const float*>(a.ws_o) + row * D + lane * PL;
+            W += wk;
+            #pragma unroll
+            for (int k = 0; k < PL; ++k) acc[k] += wk * o[k];
+        }
+    }
+    const float inv = W > 0.f ? 1.f / W : 0.f;
+    const uint64_t ob = (uint64_t(v) * a.hq + qh) * D + lane * PL;
+    #pragma unroll
+    for (int k = 0; k < PL; ++k) {
+        if constexpr (F16) static_cast<_Float16*>(a.out)[ob + k] = (_Float16)(acc[k] * inv);
+        else static_cast<__bf16*>(a.out)[ob + k] = (__bf16)(acc[k] * inv);
+    }
 }
 
 // ------------------------------------------------- decode from device CSR
@@ -3598,6 +3648,25 @@ int launch_merge(const MergeArgs& a, uint32_t q_dtype, uint32_t d, void* stream)
         case 256: return launch_merge_d<256>(a, q_dtype, s);
         default: return hipErrorInvalidValue;
     }
+}
+
+int launch_prefill_merge(const MergeArgs& a, const uint32_t* rows, uint32_t n_rows, uint32_t q_dtype, uint32_t d,
+                         void* stream) {
+    if (n_rows == 0) return hipSuccess;
+    if (q_dtype > 1) return hipErrorInvalidValue;
+    hipStream_t s = reinterpret_cast<hipStream_t>(stream);
+    const dim3 grid(uint32_t((uint64_t(n_rows) * a.hq + kWaves - 1) / kWaves)), block(kWaves * 64);
+    auto go = [&](auto f16) {
+        constexpr bool F = decltype(f16)::value;
+        switch (d) {
+            case 64: hipLaunchKernelGGL((prefill_merge_kernel<64, F>), grid, block, 0, s, a, rows, n_rows); break;
+            case 128: hipLaunchKernelGGL((prefill_merge_kernel<128, F>), grid, block, 0, s, a, rows, n_rows); break;
+            case 256: hipLaunchKernelGGL((prefill_merge_kernel<256, F>), grid, block, 0, s, a, rows, n_rows); break;
+            default: return hipErrorInvalidValue;
+        }
+        return hipGetLastError();
+    };
+    return q_dtype == 0 ? go(std::true_type{}) : go(std::false_type{});
 }
 
 int launch_merge_states(const float* o_a, const float* lse_a, const float* o_b, const float* lse_b,

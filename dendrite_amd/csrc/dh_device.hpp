@@ -55,6 +55,10 @@ constexpr uint32_t kItemTail = 1u;
 // kItemCausal (prefill): the item's rows see different numbers of tokens,
 // row_len[row's virtual sequence] each; ItemLim bounds them.
 constexpr uint32_t kItemCausal = 2u;
+// kItemSplit (prefill plans whose other items write their rows to out): the
+// item is one of several chunks of its rows and writes f32 partial states,
+// merged by prefill_merge_kernel.
+constexpr uint32_t kItemSplit = 4u;
 
 // Token range of a causal item: its pages start at token tok0 of the
 // sequence; its rows see lmin .. lmax tokens (lmin > tok0, lmax <= the
@@ -112,8 +116,9 @@ struct AttendArgs {
     // and the group items' token ranges; null for decode plans.
     const uint32_t* row_len;
     const ItemLim* item_lim;
-    // Prefill plans whose every row has one partial state: the items write
-    // the normalised rows straight to out (no merge); null otherwise.
+    // Prefill plans without chunks, or with a split tail: items other than
+    // kItemSplit ones write the normalised rows straight to out; null
+    // otherwise.
     void* out_direct;
     // Pages in the pool: a page id at or past it is read as page 0 (and, on
     // the CSR path, marks its sequence bad).  Plan ids are checked on the
@@ -232,6 +237,10 @@ int static_scratch_address(void** out);
 int launch_attend(const AttendArgs& a, uint32_t n_tasks, uint32_t q_dtype, uint32_t kv_format,
                   uint32_t head_dim, bool prefill, void* stream);
 int launch_merge(const MergeArgs& a, uint32_t q_dtype, uint32_t head_dim, void* stream);
+// Rows of a prefill plan's split blocks: n_rows virtual sequences rows[]
+// with f32 partial states in slots slot_ptr[v] .. slot_ptr[v + 1].
+int launch_prefill_merge(const MergeArgs& a, const uint32_t* rows, uint32_t n_rows, uint32_t q_dtype, uint32_t d,
+                         void* stream);
 int launch_merge_states(const float* o_a, const float* lse_a, const float* o_b,
                         const float* lse_b, float* o_out, float* lse_out, uint32_t n_rows,
                         uint32_t head_dim, void* stream);

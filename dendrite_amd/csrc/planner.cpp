@@ -12,6 +12,8 @@
 #include "planner.hpp"
 
 #include <algorithm>
+#include <functional>
+#include <queue>
 #include <unordered_map>
 
 #include "dendrite_hip.h"
@@ -607,6 +609,81 @@ int build_plan(const PlanInput& in, HostPlan& out, std::string& err) {
     return DH_OK;
 }
 
+// Cost of a prefill item in page row tiles: a page costs its tiles plus two
+// (staging); an item's start about four page pairs, and writing its f32
+// partial states about eight more.
+static uint64_t prefill_cost(uint64_t pages, uint64_t tiles) { return pages * (2 + tiles) + 80; }
+constexpr uint64_t kPrefillSplitCost = 160;
+
+struct PrefillBlock {
+    uint64_t pages, plast, tiles, rows;   // plast: a chunk may start at or below it
+};
+
+// The split of whole blocks' tail (build_prefill_plan): which blocks (the
+// `split` cheapest of `order`, cost-descending) and their chunk in pages; 0
+// blocks where no candidate ends 5 % earlier.  Items go out in cost order to
+// free workgroup slots, so a plan's end is a heaviest-first list schedule;
+// the hkv items of a block are alike, so it runs on slots / hkv columns of
+// blocks.  The last round of whole blocks leaves most of the chip idle when
+// few of them are left: 67 blocks on 64 columns take two rounds (300-900
+// new tokens over 3 750-5 000 FP8 ones, 32 / 8 heads at head_dim 128: 327 us
+// whole, 229 us with the tail split).  Split evenly, every block's rows would
+// pay for states and a merge.  Beyond eight rounds the idle share is small
+// and nothing is weighed.
+static void prefill_tail(const std::vector<PrefillBlock>& blk, const std::vector<uint32_t>& order, uint32_t slots,
+                         uint32_t hkv, uint64_t queries, uint32_t& split, uint32_t& chunk) {
+    split = chunk = 0;
+    const uint32_t n = uint32_t(order.size()), cols = std::max(1u, slots / hkv), rounds = n / cols;
+    if (rounds == 0 || rounds >= 8 || n % cols == 0) return;
+    std::vector<uint64_t> cost;
+    uint64_t sum = 0;
+    for (uint32_t i : order) {
+        cost.push_back(prefill_cost(blk[i].pages, blk[i].tiles));
+        sum += cost.back();
+    }
+    auto makespan = [&]() {   // of `cost`, in descending order
+        std::priority_queue<uint64_t, std::vector<uint64_t>, std::greater<uint64_t>> free;
+        for (uint32_t i = 0; i < cols; ++i) free.push(0);
+        uint64_t end = 0;
+        for (uint64_t c : cost) {
+            const uint64_t t = free.top() + c;
+            free.pop();
+            free.push(t);
+            end = std::max(end, t);
+        }
+        return end;
+    };
+    const uint64_t whole = makespan();
+    uint64_t best = whole - whole / 20;
+    if (sum / cols >= best) return;   // no split ends before the mean load
+    for (uint32_t r : {n % cols, n % cols + cols / 4}) {
+        if (r >= n) continue;
+        for (uint32_t ch : {16u, 32u, 64u, 128u}) {
+            cost.clear();
+            uint64_t slots_used = 0;
+            for (uint32_t i = 0; i < n; ++i) {
+                const PrefillBlock& b = blk[order[i]];
+                uint64_t p = 0, k = 0;
+                if (i >= n - r)
+                    for (; p + ch <= b.plast; p += ch, ++k) cost.push_back(prefill_cost(ch, b.tiles) + kPrefillSplitCost);
+                cost.push_back(prefill_cost(b.pages - p, b.tiles) + (k ? kPrefillSplitCost : 0));
+                if (k) slots_used += (k + 1) * b.rows;
+            }
+            std::sort(cost.begin(), cost.end(), std::greater<uint64_t>());
+            // Merge: its launch (about six page pairs) and reading the states.
+            // The workspace stays within what the whole plan asks for (f32
+            // states of half as many queries).
+            if (2 * slots_used > queries) continue;
+            const uint64_t e = makespan() + 120 + 8 * slots_used * hkv / slots;
+            if (e < best) {
+                best = e;
+                split = r;
+                chunk = ch;
+            }
+        }
+    }
+}
+
 // Prefill items: for each sequence, KV head and block of query tokens
 // (group_rows / r tokens, their r heads each a row), the KV pages the block's
 // last query sees, cut into chunks of chunk_pages.  Chunk starts stay below
@@ -676,6 +753,7 @@ int build_prefill_plan(const PrefillInput& in, HostPlan& out, std::string& err) 
     uint64_t n_blocks = 0;
     for (uint32_t b = 0; b < B; ++b) n_blocks += (in.q_len[b] + tpb - 1) / tpb;
     uint32_t chunk = in.chunk_pages;
+    const bool whole = !chunk && n_blocks * in.hkv >= 512;
     if (!chunk && n_blocks * in.hkv >= 512) {
         chunk = UINT32_MAX;
     } else if (!chunk) {
@@ -694,15 +772,40 @@ int build_prefill_plan(const PrefillInput& in, HostPlan& out, std::string& err) 
         uint32_t b, i0, i1, p0, p1;
     };
     std::vector<Piece> pieces;
+    // Blocks in (sequence, token) order; of a plan of whole blocks, those of
+    // its tail get a chunk size of their own.
+    std::vector<uint32_t> block_chunk(n_blocks, chunk);
+    if (whole) {
+        std::vector<PrefillBlock> blk;
+        bool fits = true;
+        for (uint32_t b = 0; b < B; ++b)
+            for (uint32_t i0 = 0; i0 < in.q_len[b]; i0 += tpb) {
+                const uint32_t i1 = std::min(in.q_len[b], i0 + tpb);
+                const uint64_t pend = (len_of(b, i1 - 1) + kPageSize - 1) / kPageSize;
+                blk.push_back(PrefillBlock{pend, (len_of(b, i0) - 1) / kPageSize,
+                                           ((i1 - i0) * r + kTileRows - 1) / kTileRows, i1 - i0});
+                fits = fits && pend <= kPrefillMaxChunk;
+            }
+        std::vector<uint32_t> order(blk.size());
+        for (uint32_t i = 0; i < order.size(); ++i) order[i] = i;
+        std::stable_sort(order.begin(), order.end(), [&](uint32_t x, uint32_t y) {
+            return blk[x].pages * (2 + blk[x].tiles) > blk[y].pages * (2 + blk[y].tiles);
+        });
+        uint32_t split = 0, tail_chunk = 0;
+        if (fits) prefill_tail(blk, order, in.wg_slots, in.hkv, nq, split, tail_chunk);
+        for (uint32_t i = 0; i < split; ++i) block_chunk[order[order.size() - 1 - i]] = tail_chunk;
+        out.split_tail = split > 0;
+    }
+    size_t block = 0;
     for (uint32_t b = 0; b < B; ++b) {
-        for (uint32_t i0 = 0; i0 < in.q_len[b]; i0 += tpb) {
+        for (uint32_t i0 = 0; i0 < in.q_len[b]; i0 += tpb, ++block) {
             const uint32_t i1 = std::min(in.q_len[b], i0 + tpb);
             const uint32_t lmin = len_of(b, i0), lmax = len_of(b, i1 - 1);
             const uint32_t pend = (lmax + kPageSize - 1) / kPageSize;
             const uint32_t plast = (lmin - 1) / kPageSize;       // a chunk may start at or below this page
             uint32_t p0 = 0;
             while (true) {
-                const uint64_t nx = uint64_t(p0) + chunk;
+                const uint64_t nx = uint64_t(p0) + block_chunk[block];
                 if (nx > plast || nx >= pend) {
                     pieces.push_back(Piece{b, i0, i1, p0, pend});
                     break;
@@ -721,6 +824,12 @@ int build_prefill_plan(const PrefillInput& in, HostPlan& out, std::string& err) 
     std::vector<uint32_t> count(nq, 0);
     for (const Piece& pc : pieces)
         for (uint32_t i = pc.i0; i < pc.i1; ++i) count[q_off[pc.b] + i]++;
+    // With a split tail the other blocks' rows go to out, without a slot.
+    if (out.split_tail)
+        for (uint32_t v = 0; v < nq; ++v) {
+            if (count[v] > 1) out.split_rows.push_back(v);
+            else count[v] = 0;
+        }
     out.slot_ptr.assign(nq + 1, 0);
     for (uint32_t v = 0; v < nq; ++v) out.slot_ptr[v + 1] = out.slot_ptr[v] + count[v];
     out.num_slots = out.slot_ptr[nq];
@@ -743,6 +852,7 @@ int build_prefill_plan(const PrefillInput& in, HostPlan& out, std::string& err) 
             const uint32_t v = q_off[pc.b] + i;
             out.seqslots.push_back(SeqSlot{v, cursor[v]++});
         }
+        const bool split = out.split_tail && count[q_off[pc.b] + pc.i0] > 1;
         const uint32_t tok0 = pc.p0 * kPageSize, tok_end = std::min(pc.p1 * kPageSize, in.kv_len[pc.b]);
         ItemLim lim;
         lim.tok0 = tok0;
@@ -757,7 +867,7 @@ int build_prefill_plan(const PrefillInput& in, HostPlan& out, std::string& err) 
             it.row_begin = 0;
             it.nrows = (pc.i1 - pc.i0) * r;
             it.kv_head = h;
-            it.flags = kItemCausal;
+            it.flags = kItemCausal | (split ? kItemSplit : 0u);
             it.tail_seq = 0;
             const double cost = double(it.npages) * (2.0 + (it.nrows + kTileRows - 1) / kTileRows);
             cands.push_back(Cand{cost, it, lim});

@@ -51,6 +51,10 @@ struct HostPlan {
     // (causal) item's token range.
     std::vector<uint32_t> row_len;
     std::vector<ItemLim> item_lim;
+    // Prefill plans with a split tail: the queries whose blocks are split
+    // (kItemSplit items, f32 partial states); the others have no slot.
+    bool split_tail = false;
+    std::vector<uint32_t> split_rows;
     // Decode plans, per sequence b: the chunk holding its last page, for
     // in-place updates (appending a page, replacing the last page).  Its
     // pages are pages[tail_off[b] .. + tail_n[b]) and the entries up to
@@ -75,6 +79,7 @@ struct PrefillInput {
     uint32_t group_rows = 128;
     bool causal = true;
     uint32_t chunk_pages = 0;           // 0 = chosen from the work
+    uint32_t wg_slots = 512;            // workgroups the chip holds at once
 };
 
 // Returns 0 on success, else a dh_status code with `err` set.

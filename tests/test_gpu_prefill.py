@@ -161,3 +161,21 @@ def test_prefill_items_longer_than_decode_items(backend, chunk):
          chunk_pages=chunk, seed=11)
     _run(backend, 4, 1, 128, _lib.DTYPE_BF16, _lib.KV_BF16, kv_len=[33000], q_len=[40], chunk_pages=chunk, seed=12)
     _run(backend, 8, 2, 256, _lib.DTYPE_BF16, _lib.KV_MXFP8, kv_len=[6000], q_len=[20], chunk_pages=chunk, seed=13)
+
+
+@pytest.mark.parametrize("case", [
+    (128, 8, 128, _lib.DTYPE_BF16, _lib.KV_BF16, [1500, 1490], [272, 267], True),
+    (128, 8, 128, _lib.DTYPE_F16, _lib.KV_FP8_E4M3, [1490, 1505], [261, 270], True),
+    (128, 8, 128, _lib.DTYPE_BF16, _lib.KV_MXFP8, [1100], [540], False),
+    (64, 8, 256, _lib.DTYPE_F16, _lib.KV_F16, [1500], [521], False),
+    (128, 8, 64, _lib.DTYPE_F16, _lib.KV_F16, [1300], [1040], False)],
+    ids=["bf16", "f16-fp8", "mxfp8", "d256", "d64"])
+def test_prefill_split_tail(backend, case):
+    """Plans with a few blocks more than whole rounds of the chip: the tail's
+    blocks are split, the others write out themselves.  The workspace stays
+    within what one 16-bit state per (query, head) takes."""
+    hq, hkv, d, q_dtype, fmt, kv, q, causal = case
+    plan = _run(backend, hq, hkv, d, q_dtype, fmt, kv_len=kv, q_len=q, causal=causal, seed=21)
+    tpb = (64 if d == 256 else 128) // (hq // hkv)
+    assert plan.stats()["num_items"] > hkv * sum((n + tpb - 1) // tpb for n in q)
+    assert plan.workspace().numel() <= sum(q) * hq * (2 * d + 8) + 512
