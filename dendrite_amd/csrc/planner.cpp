@@ -13,7 +13,6 @@
 
 #include <algorithm>
 #include <functional>
-#include <queue>
 #include <unordered_map>
 
 #include "dendrite_hip.h"
@@ -635,20 +634,26 @@ static void prefill_tail(const std::vector<PrefillBlock>& blk, const std::vector
     split = chunk = 0;
     const uint32_t n = uint32_t(order.size()), cols = std::max(1u, slots / hkv), rounds = n / cols;
     if (rounds == 0 || rounds >= 8 || n % cols == 0) return;
-    std::vector<uint64_t> cost;
+    std::vector<uint64_t> cost, free(cols);
+    cost.reserve(2 * n);
     uint64_t sum = 0;
     for (uint32_t i : order) {
         cost.push_back(prefill_cost(blk[i].pages, blk[i].tiles));
         sum += cost.back();
     }
     auto makespan = [&]() {   // of `cost`, in descending order
-        std::priority_queue<uint64_t, std::vector<uint64_t>, std::greater<uint64_t>> free;
-        for (uint32_t i = 0; i < cols; ++i) free.push(0);
+        std::fill(free.begin(), free.end(), 0);   // a heap, the column that is free first on top
         uint64_t end = 0;
         for (uint64_t c : cost) {
-            const uint64_t t = free.top() + c;
-            free.pop();
-            free.push(t);
+            const uint64_t t = free[0] + c;
+            uint32_t i = 0;
+            for (uint32_t k = 1; k < cols; k = 2 * i + 1) {
+                if (k + 1 < cols && free[k + 1] < free[k]) ++k;
+                if (free[k] >= t) break;
+                free[i] = free[k];
+                i = k;
+            }
+            free[i] = t;
             end = std::max(end, t);
         }
         return end;
@@ -777,6 +782,7 @@ int build_prefill_plan(const PrefillInput& in, HostPlan& out, std::string& err) 
     std::vector<uint32_t> block_chunk(n_blocks, chunk);
     if (whole) {
         std::vector<PrefillBlock> blk;
+        blk.reserve(n_blocks);
         bool fits = true;
         for (uint32_t b = 0; b < B; ++b)
             for (uint32_t i0 = 0; i0 < in.q_len[b]; i0 += tpb) {
