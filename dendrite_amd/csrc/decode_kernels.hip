@@ -3558,7 +3558,10 @@ hipError_t launch_merge_d(const MergeArgs& a, uint32_t q_dtype, hipStream_t s) {
     const uint32_t rows = a.batch * a.hq;
     if (rows == 0) return hipSuccess;
     dim3 grid((rows + 3) / 4), block(256);
-    // Rows of 17-32 states: the scalar form, one pass of 32.  Otherwise the
+    // Rows of 17-32 states: the scalar form, one pass of 32, below head_dim
+    // 256.  There its 32 rows of 8 bytes a lane take 144 registers, and the
+    // vector form's one pass is faster (8 trees of 8 leaves, 17-32 states,
+    // 16 / 2 heads, bf16: a step 32.4 -> 30.9 us).  Otherwise the
     // vector form with loads per pass for the plan's most states per row, so
     // a row loads no state twice; not known on the host (0, the CSR path):
     // chosen per row from its own count.
@@ -3568,7 +3571,7 @@ hipError_t launch_merge_d(const MergeArgs& a, uint32_t q_dtype, hipStream_t s) {
         using MS = MergeShape<D, OUT>;
         const int need = (states + MS::SPI - 1) / MS::SPI;
         if (states == 0) hipLaunchKernelGGL((merge_kernel<D, OUT, -1>), grid, block, 0, s, a);
-        else if (states > 16 && states <= 32) hipLaunchKernelGGL((merge_kernel<D, OUT, 0>), grid, block, 0, s, a);
+        else if ((D < 256 || OUT == 2) && states > 16 && states <= 32) hipLaunchKernelGGL((merge_kernel<D, OUT, 0>), grid, block, 0, s, a);
         else if (need <= 1) hipLaunchKernelGGL((merge_kernel<D, OUT, 1>), grid, block, 0, s, a);
         else if (need <= 2 && MS::MAX_NV >= 2) hipLaunchKernelGGL((merge_kernel<D, OUT, (MS::MAX_NV >= 2 ? 2 : 1)>), grid, block, 0, s, a);
         else if (need <= 4 && MS::MAX_NV >= 4) hipLaunchKernelGGL((merge_kernel<D, OUT, (MS::MAX_NV >= 4 ? 4 : 1)>), grid, block, 0, s, a);

@@ -311,3 +311,17 @@ def test_host_last_page_lengths_full_batch(backend):
     assert torch.equal(run.out.view(torch.uint8), want.view(torch.uint8))
     got = run.out.float().cpu().numpy()
     assert excess_err(got, run.reference(), w.q_dtype) <= TOL[w.q_dtype]
+
+
+@pytest.mark.parametrize("fmt", [(_lib.DTYPE_BF16, _lib.KV_BF16), (_lib.DTYPE_F16, _lib.KV_F16)],
+                         ids=["bf16", "f16"])
+@pytest.mark.parametrize("states", [16, 17, 31, 32, 33])
+def test_merge_states_at_head_dim_256(backend, fmt, states):
+    """Rows of up to 33 one-page states at head_dim 256: both sides of the
+    17..32 range, whose merge is the vector form there."""
+    tables, n = [], 0
+    for k in (states, 5, 1):
+        tables.append(list(range(n, n + k)))
+        n += k
+    w = workloads.custom(tables, 16, 2, 256, fmt[0], fmt[1], n, last_page_len=[7, 16, 1], seed=states)
+    _check(w, backend, cascade=False, private_chunk_pages=1, direct=False)
