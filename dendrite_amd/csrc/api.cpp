@@ -1231,11 +1231,11 @@ dh_status dh_decode_csr(dh_backend* be, const dh_pool* pool, const dh_attn_confi
     a.seq_bad = seq_bad;
     a.csr_nrb = nrb;
     // The group items the planning kernel writes (at most gcap) take the
-    // first workgroups; then one wave per wave item, four per workgroup,
-    // over every slot the workspace holds.  Workgroups past the call's
-    // items exit at once.
-    const uint64_t waves = slots * per_chunk;
-    e = hipError_t(dh::launch_attend(a, uint32_t(gcap + (waves + dh::kWaves - 1) / dh::kWaves), c.q_dtype,
+    // first workgroups; then one wave per wave item, four per workgroup, at
+    // most over every slot the workspace holds.  kCsrGrid workgroups take
+    // them in turns; those past the call's items exit at once.
+    const uint64_t waves = slots * per_chunk, units = gcap + (waves + dh::kWaves - 1) / dh::kWaves;
+    e = hipError_t(dh::launch_attend(a, uint32_t(std::min<uint64_t>(units, dh::kCsrGrid)), c.q_dtype,
                                      c.kv_format, c.head_dim, false, stream));
     if (e != hipSuccess) return fail(DH_EHIP, "attention launch failed: %s", hipGetErrorString(e));
 

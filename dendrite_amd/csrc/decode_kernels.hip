@@ -179,22 +179,25 @@ __device__ __forceinline__ void row_target(const AttendArgs& a, const Item& it, 
 
 // Group items of the launch: the plan's count, or on the CSR path what the
 // CSR planning kernel of this call wrote (its group items come first).
+template <bool CSR>
 __device__ __forceinline__ uint32_t group_item_count(const AttendArgs& a) {
-    return a.csr_hdr ? __builtin_amdgcn_readfirstlane(a.csr_hdr[4]) : a.n_group_items;
+    return CSR ? __builtin_amdgcn_readfirstlane(a.csr_hdr[4]) : a.n_group_items;
 }
 
-// Item of wave `wave` in a workgroup past the ng group items (AttendArgs):
+// Item of wave `wave` in unit `unit` (a workgroup's) past the ng group items:
 // on the plan path an index into the items (group items first), on the CSR
 // path the wave item's own number (csr_item).
-__device__ __forceinline__ uint32_t wave_item_index(const AttendArgs& a, int wave, uint32_t ng) {
-    return (a.csr_hdr ? 0u : ng) + (blockIdx.x - ng) * kWaves + uint32_t(wave);
+template <bool CSR>
+__device__ __forceinline__ uint32_t wave_item_index(uint32_t unit, int wave, uint32_t ng) {
+    return (CSR ? 0u : ng) + (unit - ng) * kWaves + uint32_t(wave);
 }
 
 // Wave items on the plan path: the plan's count; on the CSR path: what the
 // CSR planning kernel of this call wrote (its nodes' wave items, then one
 // per chunk of each sequence's own pages).
+template <bool CSR>
 __device__ __forceinline__ uint32_t wave_item_end(const AttendArgs& a) {
-    return a.csr_hdr ? __builtin_amdgcn_readfirstlane(a.csr_hdr[1]) + __builtin_amdgcn_readfirstlane(a.csr_hdr[6])
+    return CSR ? __builtin_amdgcn_readfirstlane(a.csr_hdr[1]) + __builtin_amdgcn_readfirstlane(a.csr_hdr[6])
                      : a.n_group_items + a.n_wave_items;
 }
 
@@ -2192,26 +2195,45 @@ __device__ __forceinline__ void wave_task_merge(const AttendArgs& a, int wave, i
     }
 }
 
-template <int D, uint32_t KVF, bool F16>
+// CSR: an instance of its own for dh_decode_csr, whose item count only the
+// device knows.  Its grid is bounded by kCsrGrid and a workgroup takes every
+// gridDim.x-th unit (a group item or four wave items).  One workgroup per
+// unit the workspace could hold launched 10 000 mostly empty ones, each
+// waiting for 66 KiB of LDS and reading the header to find out
+// (a 64-leaf f16 tree over 8 192 tokens: 48.1 -> 44.5 us a call).  The loop in the
+// plan path's kernel cost it 7-30 % (registers), hence the instance; the
+// thread index is made opaque in each round so that nothing derived from it
+// is kept in registers across rounds.
+template <int D, uint32_t KVF, bool F16, bool CSR>
 __global__ __launch_bounds__(256, D >= 256 ? 1 : 2) void attend16_kernel(AttendArgs a) {
-    const int tid = threadIdx.x, lane = tid & 63, g = lane >> 4, c = lane & 15;
-    // Wave index as a wave-uniform (scalar) value: page-list reads then go
-    // through the scalar cache and never wait on the vector loads in flight.
-    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const uint32_t ng = group_item_count(a);
-    if (blockIdx.x < ng) {
-        const Item it = a.items[blockIdx.x];
-        if constexpr ((KVF == KVF_FP8 || KVF == KVF_MX) && D == 64) group_item<D, KVF, F16>(a, it, tid, wave, g, c);
-        else if constexpr (KVF == KVF_FP8 || KVF == KVF_MX) group_item_dma8<D, KVF, F16, false>(a, it, tid, wave, g, c);
-        else group_item_dma<D, F16, false>(a, it, tid, wave, g, c);
-    } else {
-        const uint32_t idx = wave_item_index(a, wave, ng);
-        if (idx < wave_item_end(a)) {
-            const Item it = a.csr_hdr ? csr_wave_item(a, idx, ng) : a.items[idx];
-            if (it.npages) wave_item<D, KVF, F16>(a, it, g, c);   // direct tasks pad with empty items
+    const uint32_t ng = group_item_count<CSR>(a);
+    const uint32_t end = CSR ? ng + (wave_item_end<CSR>(a) + kWaves - 1) / kWaves : 0u;
+    uint32_t unit = blockIdx.x;
+    do {
+        int tid = threadIdx.x;
+        if constexpr (CSR) asm volatile("" : "+v"(tid));
+        const int lane = tid & 63, g = lane >> 4, c = lane & 15;
+        // Wave index as a wave-uniform (scalar) value: page-list reads then go
+        // through the scalar cache and never wait on the vector loads in flight.
+        const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+        if (unit < ng) {
+            const Item it = a.items[unit];
+            if constexpr ((KVF == KVF_FP8 || KVF == KVF_MX) && D == 64) group_item<D, KVF, F16>(a, it, tid, wave, g, c);
+            else if constexpr (KVF == KVF_FP8 || KVF == KVF_MX) group_item_dma8<D, KVF, F16, false>(a, it, tid, wave, g, c);
+            else group_item_dma<D, F16, false>(a, it, tid, wave, g, c);
+        } else {
+            const uint32_t idx = wave_item_index<CSR>(unit, wave, ng);
+            if (idx < wave_item_end<CSR>(a)) {
+                const Item it = CSR ? csr_wave_item(a, idx, ng) : a.items[idx];
+                if (it.npages) wave_item<D, KVF, F16>(a, it, g, c);   // direct tasks pad with empty items
+            }
+            if (!CSR && a.wave_direct) wave_task_merge<D, F16 ? 0u : 1u>(a, wave, tid & 63);
         }
-        if (a.wave_direct) wave_task_merge<D, F16 ? 0u : 1u>(a, wave, tid & 63);
-    }
+        if constexpr (CSR) {
+            unit += gridDim.x;
+            if (unit < end) __syncthreads();   // every wave is done with this unit's LDS
+        }
+    } while (CSR && unit < end);
 }
 
 // Prefill plans: causal group items only (every workgroup one item); the
@@ -2332,16 +2354,24 @@ __device__ __forceinline__ void attend32_item(const AttendArgs& a, const Item& i
     write_wave_partial<D, 1, false, true>(a, it, 0, 1, dst, m, l, O, g, c);
 }
 
-template <int D>
+// CSR: as attend16_kernel (its wave items need no LDS, so no barrier).
+template <int D, bool CSR>
 __global__ __launch_bounds__(256) void attend32_kernel(AttendArgs a) {
-    const int tid = threadIdx.x, lane = tid & 63, g = lane >> 4, c = lane & 15;
-    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const uint32_t idx = wave_item_index(a, wave, group_item_count(a));   // f32: no group items
-    if (idx < wave_item_end(a)) {
-        const Item it = a.csr_hdr ? csr_wave_item(a, idx, 0) : a.items[idx];
-        if (it.npages) attend32_item<D>(a, it, lane, g, c);   // direct tasks pad with empty items
-    }
-    if (a.wave_direct) wave_task_merge<D, 2u>(a, wave, lane);
+    const uint32_t end = CSR ? (wave_item_end<CSR>(a) + kWaves - 1) / kWaves : 0u;
+    uint32_t unit = blockIdx.x;
+    do {
+        int tid = threadIdx.x;
+        if constexpr (CSR) asm volatile("" : "+v"(tid));
+        const int lane = tid & 63, g = lane >> 4, c = lane & 15;
+        const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+        const uint32_t idx = wave_item_index<CSR>(unit, wave, group_item_count<CSR>(a));   // f32: no group items
+        if (idx < wave_item_end<CSR>(a)) {
+            const Item it = CSR ? csr_wave_item(a, idx, 0) : a.items[idx];
+            if (it.npages) attend32_item<D>(a, it, lane, g, c);   // direct tasks pad with empty items
+        }
+        if (!CSR && a.wave_direct) wave_task_merge<D, 2u>(a, wave, lane);
+        unit += gridDim.x;
+    } while (CSR && unit < end);
 }
 
 // ------------------------------------------------------------------ merge
@@ -3529,24 +3559,24 @@ hipError_t launch_prefill_d(const AttendArgs& a, uint32_t n, uint32_t q_dtype, u
     return hipGetLastError();
 }
 
-template <int D>
+template <int D, bool CSR>
 hipError_t launch_attend_d(const AttendArgs& a, uint32_t n, uint32_t q_dtype, uint32_t kvf,
                            hipStream_t s) {
     dim3 grid(n), block(kWaves * 64);
     if (q_dtype == 2 && kvf == KVF_F32) {
-        hipLaunchKernelGGL(attend32_kernel<D>, grid, block, 0, s, a);
+        hipLaunchKernelGGL((attend32_kernel<D, CSR>), grid, block, 0, s, a);
     } else if (q_dtype == 1 && kvf == KVF_BF16) {
-        hipLaunchKernelGGL((attend16_kernel<D, KVF_BF16, false>), grid, block, 0, s, a);
+        hipLaunchKernelGGL((attend16_kernel<D, KVF_BF16, false, CSR>), grid, block, 0, s, a);
     } else if (q_dtype == 1 && kvf == KVF_FP8) {
-        hipLaunchKernelGGL((attend16_kernel<D, KVF_FP8, false>), grid, block, 0, s, a);
+        hipLaunchKernelGGL((attend16_kernel<D, KVF_FP8, false, CSR>), grid, block, 0, s, a);
     } else if (q_dtype == 1 && kvf == KVF_MX) {
-        hipLaunchKernelGGL((attend16_kernel<D, KVF_MX, false>), grid, block, 0, s, a);
+        hipLaunchKernelGGL((attend16_kernel<D, KVF_MX, false, CSR>), grid, block, 0, s, a);
     } else if (q_dtype == 0 && kvf == KVF_FP8) {   // f16 queries: codes into f16, f16 MFMAs
-        hipLaunchKernelGGL((attend16_kernel<D, KVF_FP8, true>), grid, block, 0, s, a);
+        hipLaunchKernelGGL((attend16_kernel<D, KVF_FP8, true, CSR>), grid, block, 0, s, a);
     } else if (q_dtype == 0 && kvf == KVF_MX) {
-        hipLaunchKernelGGL((attend16_kernel<D, KVF_MX, true>), grid, block, 0, s, a);
+        hipLaunchKernelGGL((attend16_kernel<D, KVF_MX, true, CSR>), grid, block, 0, s, a);
     } else if (q_dtype == 0 && kvf == KVF_F16) {
-        hipLaunchKernelGGL((attend16_kernel<D, KVF_F16, true>), grid, block, 0, s, a);
+        hipLaunchKernelGGL((attend16_kernel<D, KVF_F16, true, CSR>), grid, block, 0, s, a);
     } else {
         return hipErrorInvalidValue;
     }
@@ -3615,9 +3645,12 @@ int launch_attend(const AttendArgs& a, uint32_t n_items, uint32_t q_dtype, uint3
         }
     }
     switch (d) {
-        case 64: return launch_attend_d<64>(a, n_items, q_dtype, kvf, s);
-        case 128: return launch_attend_d<128>(a, n_items, q_dtype, kvf, s);
-        case 256: return launch_attend_d<256>(a, n_items, q_dtype, kvf, s);
+        case 64: return a.csr_hdr ? launch_attend_d<64, true>(a, n_items, q_dtype, kvf, s)
+                                 : launch_attend_d<64, false>(a, n_items, q_dtype, kvf, s);
+        case 128: return a.csr_hdr ? launch_attend_d<128, true>(a, n_items, q_dtype, kvf, s)
+                                : launch_attend_d<128, false>(a, n_items, q_dtype, kvf, s);
+        case 256: return a.csr_hdr ? launch_attend_d<256, true>(a, n_items, q_dtype, kvf, s)
+                                : launch_attend_d<256, false>(a, n_items, q_dtype, kvf, s);
         default: return hipErrorInvalidValue;
     }
 }

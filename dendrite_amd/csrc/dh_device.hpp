@@ -255,6 +255,10 @@ int launch_csr_lcp(const int32_t* indptr, const int32_t* indices, uint32_t batch
 // workgroups x four waves), and its chunk sizes: 1 page up to what a wave
 // item's page-id registers hold.
 constexpr uint32_t kCsrWaveSlots = 2048;
+// Workgroups of a CSR call's attention launch: two rounds of the 512 that fit
+// the chip, so that a slot freed early still takes new work; the units past
+// them (the shortest chunks, last in dispatch order) go to workgroups again.
+constexpr uint32_t kCsrGrid = 1024;
 constexpr uint32_t kCsrMinChunk = 1, kCsrMaxChunk = uint32_t(kWaveIdRegs) * 64;
 }  // namespace dh
 }
