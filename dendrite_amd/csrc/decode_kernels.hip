@@ -181,15 +181,15 @@ __device__ __forceinline__ void row_target(const AttendArgs& a, const Item& it, 
 // CSR planning kernel of this call wrote (its group items come first).
 template <bool CSR>
 __device__ __forceinline__ uint32_t group_item_count(const AttendArgs& a) {
-    return CSR ? __builtin_amdgcn_readfirstlane(a.csr_hdr[4]) : a.n_group_items;
+    return CSR || a.csr_hdr ? __builtin_amdgcn_readfirstlane(a.csr_hdr[4]) : a.n_group_items;
 }
 
 // Item of wave `wave` in unit `unit` (a workgroup's) past the ng group items:
 // on the plan path an index into the items (group items first), on the CSR
 // path the wave item's own number (csr_item).
 template <bool CSR>
-__device__ __forceinline__ uint32_t wave_item_index(uint32_t unit, int wave, uint32_t ng) {
-    return (CSR ? 0u : ng) + (unit - ng) * kWaves + uint32_t(wave);
+__device__ __forceinline__ uint32_t wave_item_index(const AttendArgs& a, uint32_t unit, int wave, uint32_t ng) {
+    return (CSR || a.csr_hdr ? 0u : ng) + (unit - ng) * kWaves + uint32_t(wave);
 }
 
 // Wave items on the plan path: the plan's count; on the CSR path: what the
@@ -197,7 +197,7 @@ __device__ __forceinline__ uint32_t wave_item_index(uint32_t unit, int wave, uin
 // per chunk of each sequence's own pages).
 template <bool CSR>
 __device__ __forceinline__ uint32_t wave_item_end(const AttendArgs& a) {
-    return CSR ? __builtin_amdgcn_readfirstlane(a.csr_hdr[1]) + __builtin_amdgcn_readfirstlane(a.csr_hdr[6])
+    return CSR || a.csr_hdr ? __builtin_amdgcn_readfirstlane(a.csr_hdr[1]) + __builtin_amdgcn_readfirstlane(a.csr_hdr[6])
                      : a.n_group_items + a.n_wave_items;
 }
 
@@ -2195,23 +2195,45 @@ __device__ __forceinline__ void wave_task_merge(const AttendArgs& a, int wave, i
     }
 }
 
-// CSR: an instance of its own for dh_decode_csr, whose item count only the
-// device knows.  Its grid is bounded by kCsrGrid and a workgroup takes every
+template <int D, uint32_t KVF, bool F16>
+__global__ __launch_bounds__(256, D >= 256 ? 1 : 2) void attend16_kernel(AttendArgs a) {
+    const int tid = threadIdx.x, lane = tid & 63, g = lane >> 4, c = lane & 15;
+    // Wave index as a wave-uniform (scalar) value: page-list reads then go
+    // through the scalar cache and never wait on the vector loads in flight.
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const uint32_t ng = group_item_count<false>(a);
+    if (blockIdx.x < ng) {
+        const Item it = a.items[blockIdx.x];
+        if constexpr ((KVF == KVF_FP8 || KVF == KVF_MX) && D == 64) group_item<D, KVF, F16>(a, it, tid, wave, g, c);
+        else if constexpr (KVF == KVF_FP8 || KVF == KVF_MX) group_item_dma8<D, KVF, F16, false>(a, it, tid, wave, g, c);
+        else group_item_dma<D, F16, false>(a, it, tid, wave, g, c);
+    } else {
+        const uint32_t idx = wave_item_index<false>(a, blockIdx.x, wave, ng);
+        if (idx < wave_item_end<false>(a)) {
+            const Item it = a.csr_hdr ? csr_wave_item(a, idx, ng) : a.items[idx];
+            if (it.npages) wave_item<D, KVF, F16>(a, it, g, c);   // direct tasks pad with empty items
+        }
+        if (a.wave_direct) wave_task_merge<D, F16 ? 0u : 1u>(a, wave, tid & 63);
+    }
+}
+
+// The attention kernel of dh_decode_csr, whose item count only the device
+// knows.  Its grid is bounded by kCsrGrid and a workgroup takes every
 // gridDim.x-th unit (a group item or four wave items).  One workgroup per
 // unit the workspace could hold launched 10 000 mostly empty ones, each
 // waiting for 66 KiB of LDS and reading the header to find out
 // (a 64-leaf f16 tree over 8 192 tokens: 48.1 -> 44.5 us a call).  The loop in the
-// plan path's kernel cost it 7-30 % (registers), hence the instance; the
+// plan path's kernel cost it 7-30 % (registers), hence a kernel of its own; the
 // thread index is made opaque in each round so that nothing derived from it
 // is kept in registers across rounds.
-template <int D, uint32_t KVF, bool F16, bool CSR>
-__global__ __launch_bounds__(256, D >= 256 ? 1 : 2) void attend16_kernel(AttendArgs a) {
-    const uint32_t ng = group_item_count<CSR>(a);
-    const uint32_t end = CSR ? ng + (wave_item_end<CSR>(a) + kWaves - 1) / kWaves : 0u;
+template <int D, uint32_t KVF, bool F16>
+__global__ __launch_bounds__(256, D >= 256 ? 1 : 2) void csr_attend16_kernel(AttendArgs a) {
+    const uint32_t ng = group_item_count<true>(a);
+    const uint32_t end = ng + (wave_item_end<true>(a) + kWaves - 1) / kWaves;
     uint32_t unit = blockIdx.x;
     do {
         int tid = threadIdx.x;
-        if constexpr (CSR) asm volatile("" : "+v"(tid));
+        asm volatile("" : "+v"(tid));
         const int lane = tid & 63, g = lane >> 4, c = lane & 15;
         // Wave index as a wave-uniform (scalar) value: page-list reads then go
         // through the scalar cache and never wait on the vector loads in flight.
@@ -2222,18 +2244,15 @@ __global__ __launch_bounds__(256, D >= 256 ? 1 : 2) void attend16_kernel(AttendA
             else if constexpr (KVF == KVF_FP8 || KVF == KVF_MX) group_item_dma8<D, KVF, F16, false>(a, it, tid, wave, g, c);
             else group_item_dma<D, F16, false>(a, it, tid, wave, g, c);
         } else {
-            const uint32_t idx = wave_item_index<CSR>(unit, wave, ng);
-            if (idx < wave_item_end<CSR>(a)) {
-                const Item it = CSR ? csr_wave_item(a, idx, ng) : a.items[idx];
-                if (it.npages) wave_item<D, KVF, F16>(a, it, g, c);   // direct tasks pad with empty items
+            const uint32_t idx = wave_item_index<true>(a, unit, wave, ng);
+            if (idx < wave_item_end<true>(a)) {
+                const Item it = csr_wave_item(a, idx, ng);
+                if (it.npages) wave_item<D, KVF, F16>(a, it, g, c);
             }
-            if (!CSR && a.wave_direct) wave_task_merge<D, F16 ? 0u : 1u>(a, wave, tid & 63);
         }
-        if constexpr (CSR) {
-            unit += gridDim.x;
-            if (unit < end) __syncthreads();   // every wave is done with this unit's LDS
-        }
-    } while (CSR && unit < end);
+        unit += gridDim.x;
+        if (unit < end) __syncthreads();   // every wave is done with this unit's LDS
+    } while (unit < end);
 }
 
 // Prefill plans: causal group items only (every workgroup one item); the
@@ -2354,24 +2373,35 @@ __device__ __forceinline__ void attend32_item(const AttendArgs& a, const Item& i
     write_wave_partial<D, 1, false, true>(a, it, 0, 1, dst, m, l, O, g, c);
 }
 
-// CSR: as attend16_kernel (its wave items need no LDS, so no barrier).
-template <int D, bool CSR>
+template <int D>
 __global__ __launch_bounds__(256) void attend32_kernel(AttendArgs a) {
-    const uint32_t end = CSR ? (wave_item_end<CSR>(a) + kWaves - 1) / kWaves : 0u;
+    const int tid = threadIdx.x, lane = tid & 63, g = lane >> 4, c = lane & 15;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const uint32_t idx = wave_item_index<false>(a, blockIdx.x, wave, group_item_count<false>(a));   // f32: no group items
+    if (idx < wave_item_end<false>(a)) {
+        const Item it = a.csr_hdr ? csr_wave_item(a, idx, 0) : a.items[idx];
+        if (it.npages) attend32_item<D>(a, it, lane, g, c);   // direct tasks pad with empty items
+    }
+    if (a.wave_direct) wave_task_merge<D, 2u>(a, wave, lane);
+}
+
+// As csr_attend16_kernel (its wave items need no LDS, so no barrier).
+template <int D>
+__global__ __launch_bounds__(256) void csr_attend32_kernel(AttendArgs a) {
+    const uint32_t end = (wave_item_end<true>(a) + kWaves - 1) / kWaves;
     uint32_t unit = blockIdx.x;
     do {
         int tid = threadIdx.x;
-        if constexpr (CSR) asm volatile("" : "+v"(tid));
+        asm volatile("" : "+v"(tid));
         const int lane = tid & 63, g = lane >> 4, c = lane & 15;
         const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-        const uint32_t idx = wave_item_index<CSR>(unit, wave, group_item_count<CSR>(a));   // f32: no group items
-        if (idx < wave_item_end<CSR>(a)) {
-            const Item it = CSR ? csr_wave_item(a, idx, 0) : a.items[idx];
-            if (it.npages) attend32_item<D>(a, it, lane, g, c);   // direct tasks pad with empty items
+        const uint32_t idx = wave_item_index<true>(a, unit, wave, group_item_count<true>(a));   // f32: no group items
+        if (idx < wave_item_end<true>(a)) {
+            const Item it = csr_wave_item(a, idx, 0);
+            if (it.npages) attend32_item<D>(a, it, lane, g, c);
         }
-        if (!CSR && a.wave_direct) wave_task_merge<D, 2u>(a, wave, lane);
         unit += gridDim.x;
-    } while (CSR && unit < end);
+    } while (unit < end);
 }
 
 // ------------------------------------------------------------------ merge
@@ -3563,20 +3593,21 @@ template <int D, bool CSR>
 hipError_t launch_attend_d(const AttendArgs& a, uint32_t n, uint32_t q_dtype, uint32_t kvf,
                            hipStream_t s) {
     dim3 grid(n), block(kWaves * 64);
+    auto go = [&](void (*kernel)(AttendArgs)) { hipLaunchKernelGGL(kernel, grid, block, 0, s, a); };
     if (q_dtype == 2 && kvf == KVF_F32) {
-        hipLaunchKernelGGL((attend32_kernel<D, CSR>), grid, block, 0, s, a);
+        go(CSR ? csr_attend32_kernel<D> : attend32_kernel<D>);
     } else if (q_dtype == 1 && kvf == KVF_BF16) {
-        hipLaunchKernelGGL((attend16_kernel<D, KVF_BF16, false, CSR>), grid, block, 0, s, a);
+        go(CSR ? csr_attend16_kernel<D, KVF_BF16, false> : attend16_kernel<D, KVF_BF16, false>);
     } else if (q_dtype == 1 && kvf == KVF_FP8) {
-        hipLaunchKernelGGL((attend16_kernel<D, KVF_FP8, false, CSR>), grid, block, 0, s, a);
+        go(CSR ? csr_attend16_kernel<D, KVF_FP8, false> : attend16_kernel<D, KVF_FP8, false>);
     } else if (q_dtype == 1 && kvf == KVF_MX) {
-        hipLaunchKernelGGL((attend16_kernel<D, KVF_MX, false, CSR>), grid, block, 0, s, a);
+        go(CSR ? csr_attend16_kernel<D, KVF_MX, false> : attend16_kernel<D, KVF_MX, false>);
     } else if (q_dtype == 0 && kvf == KVF_FP8) {   // f16 queries: codes into f16, f16 MFMAs
-        hipLaunchKernelGGL((attend16_kernel<D, KVF_FP8, true, CSR>), grid, block, 0, s, a);
+        go(CSR ? csr_attend16_kernel<D, KVF_FP8, true> : attend16_kernel<D, KVF_FP8, true>);
     } else if (q_dtype == 0 && kvf == KVF_MX) {
-        hipLaunchKernelGGL((attend16_kernel<D, KVF_MX, true, CSR>), grid, block, 0, s, a);
+        go(CSR ? csr_attend16_kernel<D, KVF_MX, true> : attend16_kernel<D, KVF_MX, true>);
     } else if (q_dtype == 0 && kvf == KVF_F16) {
-        hipLaunchKernelGGL((attend16_kernel<D, KVF_F16, true, CSR>), grid, block, 0, s, a);
+        go(CSR ? csr_attend16_kernel<D, KVF_F16, true> : attend16_kernel<D, KVF_F16, true>);
     } else {
         return hipErrorInvalidValue;
     }
