@@ -1230,13 +1230,13 @@ dh_status dh_decode_csr(dh_backend* be, const dh_pool* pool, const dh_attn_confi
     a.csr_hdr = reinterpret_cast<const uint32_t*>(hdr);
     a.seq_bad = seq_bad;
     a.csr_nrb = nrb;
-    // The group items the planning kernel writes (at most gcap) take the
-    // first workgroups; then one wave per wave item, four per workgroup, at
-    // most over every slot the workspace holds.  kCsrGrid workgroups take
-    // them in turns; those past the call's items exit at once.
+    // Units of work: the group items the planning kernel writes (at most
+    // gcap), then one wave per wave item, four per workgroup, at most over
+    // every slot the workspace holds.  A bounded number of workgroups takes
+    // them (kCsrExtraGrid); those past the call's units exit at once.
     const uint64_t waves = slots * per_chunk, units = gcap + (waves + dh::kWaves - 1) / dh::kWaves;
-    e = hipError_t(dh::launch_attend(a, uint32_t(std::min<uint64_t>(units, dh::kCsrGrid)), c.q_dtype,
-                                     c.kv_format, c.head_dim, false, stream));
+    a.csr_grid = uint32_t(std::min(units, uint64_t(batch) * per_chunk / dh::kWaves + dh::kCsrExtraGrid));
+    e = hipError_t(dh::launch_attend(a, a.csr_grid, c.q_dtype, c.kv_format, c.head_dim, false, stream));
     if (e != hipSuccess) return fail(DH_EHIP, "attention launch failed: %s", hipGetErrorString(e));
 
     dh::MergeArgs m{};

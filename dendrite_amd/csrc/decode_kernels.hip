@@ -2217,42 +2217,63 @@ __global__ __launch_bounds__(256, D >= 256 ? 1 : 2) void attend16_kernel(AttendA
     }
 }
 
-// The attention kernel of dh_decode_csr, whose item count only the device
-// knows.  Its grid is bounded by kCsrGrid and a workgroup takes every
-// gridDim.x-th unit (a group item or four wave items).  One workgroup per
-// unit the workspace could hold launched 10 000 mostly empty ones, each
-// waiting for 66 KiB of LDS and reading the header to find out
-// (a 64-leaf f16 tree over 8 192 tokens: 48.1 -> 44.5 us a call).  The loop in the
-// plan path's kernel cost it 7-30 % (registers), hence a kernel of its own; the
-// thread index is made opaque in each round so that nothing derived from it
-// is kept in registers across rounds.
+// The kernel's arguments (the first and only parameter), read anew from the
+// kernel argument segment through a pointer the compiler cannot see through:
+// neither they nor anything derived from them is held in registers up to the
+// call.
+__device__ __forceinline__ const AttendArgs& fresh_args() {
+    auto p = __builtin_amdgcn_kernarg_segment_ptr();
+    asm volatile("" : "+s"(p));
+    return *(const AttendArgs*)p;
+}
+
+// One unit of a CSR call: a group item, or past those ng four wave items.
+template <int D, uint32_t KVF, bool F16>
+__device__ __forceinline__ void csr_unit16(const AttendArgs& a, uint32_t unit, uint32_t ng, int tid) {
+    const int lane = tid & 63, g = lane >> 4, c = lane & 15;
+    // Wave index as a wave-uniform (scalar) value: page-list reads then go
+    // through the scalar cache and never wait on the vector loads in flight.
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    if (unit < ng) {
+        const Item it = a.items[unit];
+        if constexpr ((KVF == KVF_FP8 || KVF == KVF_MX) && D == 64) group_item<D, KVF, F16>(a, it, tid, wave, g, c);
+        else if constexpr (KVF == KVF_FP8 || KVF == KVF_MX) group_item_dma8<D, KVF, F16, false>(a, it, tid, wave, g, c);
+        else group_item_dma<D, F16, false>(a, it, tid, wave, g, c);
+    } else {
+        const uint32_t idx = wave_item_index<true>(a, unit, wave, ng);
+        if (idx < wave_item_end<true>(a)) {
+            const Item it = csr_wave_item(a, idx, ng);
+            if (it.npages) wave_item<D, KVF, F16>(a, it, g, c);
+        }
+    }
+}
+
+// The attention kernel of dh_decode_csr, whose unit count only the device
+// knows.  Workgroup b of csr_grid takes unit b and then, where the call has
+// more units than that, every csr_grid-th one.  One workgroup per unit the
+// workspace could hold launched 10 000 mostly empty ones for a 64-leaf f16
+// tree over 8 192 tokens, each waiting for 66 KiB of LDS to find that it had
+// nothing to do: 47.8 us a call, 43.2 with the bounded grid.
+// The first unit stands before the loop, in code of its own: a single loop
+// body, its arguments held across the rounds, spilled 25-63 scalar registers
+// into VGPR lanes and slowed most calls (48 ragged bf16 sequences: 246.7 ->
+// 248.9 us; 96 f32 ones: 239.7 -> 244.4).  The loop reads its arguments and
+// the thread index anew in each round (fresh_args) for the same reason.  Only
+// group items use LDS, and they come first: no barrier stands between others.
 template <int D, uint32_t KVF, bool F16>
 __global__ __launch_bounds__(256, D >= 256 ? 1 : 2) void csr_attend16_kernel(AttendArgs a) {
+    const int tid0 = threadIdx.x;
+    const uint32_t first = blockIdx.x, next = first + a.csr_grid;
     const uint32_t ng = group_item_count<true>(a);
     const uint32_t end = ng + (wave_item_end<true>(a) + kWaves - 1) / kWaves;
-    uint32_t unit = blockIdx.x;
-    do {
-        int tid = threadIdx.x;
+    csr_unit16<D, KVF, F16>(a, first, ng, tid0);
+    #pragma unroll 1
+    for (uint32_t unit = next; unit < end; unit += fresh_args().csr_grid) {
+        if (unit < ng) __syncthreads();   // every wave is done with the last group item's LDS
+        int tid = tid0;
         asm volatile("" : "+v"(tid));
-        const int lane = tid & 63, g = lane >> 4, c = lane & 15;
-        // Wave index as a wave-uniform (scalar) value: page-list reads then go
-        // through the scalar cache and never wait on the vector loads in flight.
-        const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-        if (unit < ng) {
-            const Item it = a.items[unit];
-            if constexpr ((KVF == KVF_FP8 || KVF == KVF_MX) && D == 64) group_item<D, KVF, F16>(a, it, tid, wave, g, c);
-            else if constexpr (KVF == KVF_FP8 || KVF == KVF_MX) group_item_dma8<D, KVF, F16, false>(a, it, tid, wave, g, c);
-            else group_item_dma<D, F16, false>(a, it, tid, wave, g, c);
-        } else {
-            const uint32_t idx = wave_item_index<true>(a, unit, wave, ng);
-            if (idx < wave_item_end<true>(a)) {
-                const Item it = csr_wave_item(a, idx, ng);
-                if (it.npages) wave_item<D, KVF, F16>(a, it, g, c);
-            }
-        }
-        unit += gridDim.x;
-        if (unit < end) __syncthreads();   // every wave is done with this unit's LDS
-    } while (unit < end);
+        csr_unit16<D, KVF, F16>(fresh_args(), unit, ng, tid);
+    }
 }
 
 // Prefill plans: causal group items only (every workgroup one item); the
@@ -2385,23 +2406,30 @@ __global__ __launch_bounds__(256) void attend32_kernel(AttendArgs a) {
     if (a.wave_direct) wave_task_merge<D, 2u>(a, wave, lane);
 }
 
-// As csr_attend16_kernel (its wave items need no LDS, so no barrier).
+// As csr_unit16 and csr_attend16_kernel (f32: wave items only, no LDS).
+template <int D>
+__device__ __forceinline__ void csr_unit32(const AttendArgs& a, uint32_t unit, int tid) {
+    const int lane = tid & 63, g = lane >> 4, c = lane & 15;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const uint32_t idx = wave_item_index<true>(a, unit, wave, group_item_count<true>(a));
+    if (idx < wave_item_end<true>(a)) {
+        const Item it = csr_wave_item(a, idx, 0);
+        if (it.npages) attend32_item<D>(a, it, lane, g, c);
+    }
+}
+
 template <int D>
 __global__ __launch_bounds__(256) void csr_attend32_kernel(AttendArgs a) {
+    const int tid0 = threadIdx.x;
+    const uint32_t first = blockIdx.x, next = first + a.csr_grid;
     const uint32_t end = (wave_item_end<true>(a) + kWaves - 1) / kWaves;
-    uint32_t unit = blockIdx.x;
-    do {
-        int tid = threadIdx.x;
+    csr_unit32<D>(a, first, tid0);
+    #pragma unroll 1
+    for (uint32_t unit = next; unit < end; unit += fresh_args().csr_grid) {
+        int tid = tid0;
         asm volatile("" : "+v"(tid));
-        const int lane = tid & 63, g = lane >> 4, c = lane & 15;
-        const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-        const uint32_t idx = wave_item_index<true>(a, unit, wave, group_item_count<true>(a));   // f32: no group items
-        if (idx < wave_item_end<true>(a)) {
-            const Item it = csr_wave_item(a, idx, 0);
-            if (it.npages) attend32_item<D>(a, it, lane, g, c);
-        }
-        unit += gridDim.x;
-    } while (unit < end);
+        csr_unit32<D>(fresh_args(), unit, tid);
+    }
 }
 
 // ------------------------------------------------------------------ merge

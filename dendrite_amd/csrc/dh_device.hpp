@@ -132,6 +132,7 @@ struct AttendArgs {
     const uint32_t* csr_hdr;      // CsrHeader
     uint32_t* seq_bad;            // [B] set to 1 for a sequence with a bad page id
     uint32_t csr_nrb;             // row blocks of 16 per (chunk, kv head)
+    uint32_t csr_grid;            // workgroups of the launch
     // Cascade on the CSR path: per sequence, its leading pages read by group
     // items (bits 0..15) and the partial-state slots those take (bits
     // 16..31); its wave items cover the rest.  Null: no cascade.
@@ -255,10 +256,15 @@ int launch_csr_lcp(const int32_t* indptr, const int32_t* indices, uint32_t batch
 // workgroups x four waves), and its chunk sizes: 1 page up to what a wave
 // item's page-id registers hold.
 constexpr uint32_t kCsrWaveSlots = 2048;
-// Workgroups of a CSR call's attention launch: two rounds of the 512 that fit
-// the chip, so that a slot freed early still takes new work; the units past
-// them (the shortest chunks, last in dispatch order) go to workgroups again.
-constexpr uint32_t kCsrGrid = 1024;
+// Workgroups of a CSR call's attention launch beyond one per four (KV head,
+// row block)s of its sequences, which have a wave item each where they hold
+// pages: room for the group items and for the extra chunks that give the chip
+// its wave slots.  The hardware hands workgroups to the first free slot; the
+// units past the grid go to fixed ones (csr_attend16_kernel).  1 500 sequences
+// of 20-700 tokens, 3 000 units: 442 us, and 449 with 1 024 workgroups in
+// all.  A 64-leaf tree of 450 units: 43.2 us up to 2 048 workgroups, 46.9
+// with 4 096.
+constexpr uint32_t kCsrExtraGrid = 1024;
 constexpr uint32_t kCsrMinChunk = 1, kCsrMaxChunk = uint32_t(kWaveIdRegs) * 64;
 }  // namespace dh
 }
