@@ -760,8 +760,7 @@ dh_status dh_plan_create_prefill(dh_backend* be, const dh_attn_config* cfg, cons
     in.group_rows = uint32_t(dh::group_rows(false, int(cfg->head_dim)));
     in.causal = causal != 0;
     in.chunk_pages = chunk_pages;
-    // Workgroups per CU by the kernel's LDS: 40 KiB, 72 KiB or more than 80.
-    in.wg_slots = 256u * (cfg->head_dim == 64 ? 4u : cfg->head_dim == 128 ? 2u : 1u);
+    in.wg_slots = dh::prefill_slots(int(cfg->head_dim));
     dh::HostPlan hp;
     std::string err;
     const int rc = dh::build_prefill_plan(in, hp, err);

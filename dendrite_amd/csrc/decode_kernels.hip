@@ -999,10 +999,13 @@ struct DmaCfg {
     static constexpr int RB = 2 * D;                  // bytes per row
     static constexpr int PLANE = kPageSize * RB;
     static constexpr int PAGE = 2 * PLANE;            // 4, 8 or 16 KiB
-    // Four page pairs.  At D = 64 a 64 KiB ring of eight left two workgroups
-    // a CU; four pairs with the prefill id list are 40 KiB, four workgroups
-    // (12 prompts of 37-1 500 tokens, 32 / 4 heads, f16: 76.2 -> 73.2 us;
-    // decode items of 32 pages the same).
+    // Four page pairs.  At D = 64 eight pairs (64 KiB) are slower: prefill
+    // of 12 prompts of 37-1 500 tokens, 32 / 4 heads, f16, 76.2 us against
+    // 73.2.  Registers hold that kernel at two workgroups a CU either way, but
+    // its code, unrolled over the ring's slots, was as long as the 64 KiB
+    // instruction cache two CUs share, and is 37 KiB.  The decode kernel, of
+    // fewer registers, goes from two workgroups a CU to three (a forked batch
+    // of 32-page items: the same time).
     static constexpr int RING = D * 512;              // LDS bytes of the ring
     static constexpr int NP = RING / (2 * PAGE);      // page pairs in the ring
     static constexpr int DPP = PAGE / (kWaves * 64 * 16);   // wave loads per thread per page

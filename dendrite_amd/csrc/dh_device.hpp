@@ -38,6 +38,10 @@ DH_HOST_DEVICE constexpr int group_tiles16(int head_dim) { return head_dim == 25
 DH_HOST_DEVICE constexpr int group_rows(bool fp8_kv, int head_dim) {
     return kWaves * ((fp8_kv && head_dim == 64) ? kGroupTiles8 : group_tiles16(head_dim)) * kTileRows;
 }
+// Workgroups of the prefill kernel the chip holds at once, on 256 CUs: two a
+// CU at head_dim 64 (178 registers: two waves a SIMD; its 40 KiB of LDS would
+// allow four) and 128 (254-256 registers, 72-76 KiB), one at 256 (136-140 KiB).
+DH_HOST_DEVICE constexpr uint32_t prefill_slots(int head_dim) { return 256u * (head_dim == 256 ? 1u : 2u); }
 
 // One attention work item (32 bytes): a run of pages of one segment chunk,
 // one KV head and a block of query rows.

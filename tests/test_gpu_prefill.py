@@ -168,8 +168,9 @@ def test_prefill_items_longer_than_decode_items(backend, chunk):
     (128, 8, 128, _lib.DTYPE_F16, _lib.KV_FP8_E4M3, [1490, 1505], [261, 270], True),
     (128, 8, 128, _lib.DTYPE_BF16, _lib.KV_MXFP8, [1100], [540], False),
     (64, 8, 256, _lib.DTYPE_F16, _lib.KV_F16, [1500], [521], False),
-    (128, 8, 64, _lib.DTYPE_F16, _lib.KV_F16, [1300], [1040], False)],
-    ids=["bf16", "f16-fp8", "mxfp8", "d256", "d64"])
+    (128, 8, 64, _lib.DTYPE_F16, _lib.KV_F16, [1300], [1040], False),
+    (128, 8, 64, _lib.DTYPE_F16, _lib.KV_F16, [1500], [536], True)],
+    ids=["bf16", "f16-fp8", "mxfp8", "d256", "d64", "d64-one-round"])
 def test_prefill_split_tail(backend, case):
     """Plans with a few blocks more than whole rounds of the chip: the tail's
     blocks are split, the others write out themselves.  The workspace stays

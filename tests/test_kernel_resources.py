@@ -82,3 +82,18 @@ def test_device_table_kernels_hold_as_many_waves(name):
     assert waves_per_simd(table) >= waves_per_simd(plan)
     assert table[".private_segment_fixed_size"] == 0
     assert table[".vgpr_spill_count"] == 0 and table[".sgpr_spill_count"] <= 8
+
+
+@pytest.mark.parametrize("d", [64, 128, 256])
+def test_prefill_slots_are_what_the_kernels_allow(d):
+    """prefill_slots (dh_device.hpp), which the prefill planner schedules
+    against, is what every prefill kernel of that head_dim allows by its
+    registers and its share of a CU's 160 KiB of LDS."""
+    with open(os.path.join(dbuild.CSRC, "dh_device.hpp")) as f:
+        rule = re.search(r"prefill_slots\(int head_dim\) { return 256u \* \(head_dim == 256 \? (\d)u : (\d)u\); }",
+                         f.read())
+    per_cu = int(rule.group(1 if d == 256 else 2))
+    found = [k for n, k in kernels().items() if n.startswith(f"prefill16_kernel<{d},")]
+    assert len(found) == (2 if d == 64 else 6)
+    for k in found:
+        assert min(waves_per_simd(k), 160 * 1024 // k[".group_segment_fixed_size"]) == per_cu
