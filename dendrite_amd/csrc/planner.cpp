@@ -618,75 +618,106 @@ struct PrefillBlock {
     uint64_t pages, plast, tiles, rows;   // plast: a chunk may start at or below it
 };
 
-// The split of whole blocks' tail (build_prefill_plan): which blocks (the
-// `split` cheapest of `order`, cost-descending) and their chunk in pages; 0
-// blocks where no candidate ends 5 % earlier.  Items go out in cost order to
-// free workgroup slots, so a plan's end is a heaviest-first list schedule;
-// the hkv items of a block are alike, so it runs on slots / hkv columns of
-// blocks.  The last round of whole blocks leaves most of the chip idle when
-// few of them are left: 67 blocks on 64 columns take two rounds (300-900
-// new tokens over 3 750-5 000 FP8 ones, 32 / 8 heads at head_dim 128: 327 us
-// whole, 229 us with the tail split).  Split evenly, every block's rows would
-// pay for states and a merge.  Beyond eight rounds the idle share is small
-// and nothing is weighed.
-static void prefill_tail(const std::vector<PrefillBlock>& blk, const std::vector<uint32_t>& order, uint32_t slots,
-                         uint32_t hkv, uint64_t queries, uint32_t& split, uint32_t& chunk) {
-    split = chunk = 0;
-    const uint32_t n = uint32_t(order.size()), cols = std::max(1u, slots / hkv), rounds = n / cols;
-    if (rounds == 0 || rounds >= 8 || n % cols == 0) return;
-    std::vector<uint64_t> cost, free(cols);
-    cost.reserve(2 * n);
-    uint64_t sum = 0;
-    for (uint32_t i : order) {
-        cost.push_back(prefill_cost(blk[i].pages, blk[i].tiles));
-        sum += cost.back();
-    }
-    auto makespan = [&]() {   // of `cost`, in descending order
-        std::fill(free.begin(), free.end(), 0);   // a heap, the column that is free first on top
-        uint64_t end = 0;
-        for (uint64_t c : cost) {
-            const uint64_t t = free[0] + c;
-            uint32_t i = 0;
-            for (uint32_t k = 1; k < cols; k = 2 * i + 1) {
-                if (k + 1 < cols && free[k + 1] < free[k]) ++k;
-                if (free[k] >= t) break;
-                free[i] = free[k];
-                i = k;
-            }
-            free[i] = t;
-            end = std::max(end, t);
+// End of the heaviest-first list schedule of `cost` (descending, at least
+// `columns` of them) on `columns` columns, or at least `limit`, where it stops.
+static uint64_t prefill_makespan(const std::vector<uint64_t>& cost, uint32_t columns, uint64_t limit) {
+    // A heap, the column that is free first on top; the first round, one item
+    // a column, stands in heap order when written from its cheapest on.
+    std::vector<uint64_t> free(cost.rend() - columns, cost.rend());
+    uint64_t end = cost[0];
+    for (size_t j = columns; j < cost.size() && end < limit; ++j) {
+        const uint64_t t = free[0] + cost[j];
+        uint32_t i = 0;
+        for (uint32_t k = 1; k < columns; k = 2 * i + 1) {
+            if (k + 1 < columns && free[k + 1] < free[k]) ++k;
+            if (free[k] >= t) break;
+            free[i] = free[k];
+            i = k;
         }
-        return end;
+        free[i] = t;
+        end = std::max(end, t);
+    }
+    return end;
+}
+
+// The split of whole blocks' tail (build_prefill_plan): the blocks to split
+// (the cheapest ones) and their chunk in pages; none where no candidate ends
+// 5 % earlier.  Items go out in cost order to free workgroup slots, so a
+// plan's end is a heaviest-first list schedule; the hkv items of a block are
+// alike, so it runs on `cols` = slots / hkv columns of blocks.  The last round
+// of whole blocks leaves most of the chip idle when few of them are left: 67
+// blocks on 64 columns take two rounds (300-900 new tokens over 3 750-5 000
+// FP8 ones, 32 / 8 heads at head_dim 128: 327 us whole, 229 us with the tail
+// split).  Split evenly, every block's rows would pay for states and a merge.
+// Candidates are turned down by what needs no schedule first: the states they
+// take, then their mean load (3 000 tokens over 28 K, 32 / 1 heads, where none
+// is left: a plan takes 835 us with every candidate's schedule, 47 us so, 46 us
+// without the search).
+static std::vector<uint32_t> prefill_tail(const std::vector<PrefillBlock>& blk, uint32_t cols, uint32_t slots,
+                                          uint32_t hkv, uint64_t queries, uint32_t& chunk) {
+    const size_t n = blk.size(), rem = n % cols;
+    // Blocks by cost, descending, equal ones in order: cost and ~index in a key.
+    std::vector<uint64_t> key(n);
+    for (size_t i = 0; i < n; ++i) key[i] = (blk[i].pages * (2 + blk[i].tiles)) << 32 | (UINT32_MAX - uint32_t(i));
+    auto block = [&](uint64_t k) -> const PrefillBlock& { return blk[UINT32_MAX - uint32_t(k)]; };
+    const size_t rmax = rem + cols / 4 < n ? rem + cols / 4 : rem;
+    std::nth_element(key.begin(), key.end() - rmax, key.end(), std::greater<uint64_t>());
+    std::sort(key.end() - rmax, key.end(), std::greater<uint64_t>());
+    struct Candidate {
+        size_t r;                  // blocks split
+        uint32_t shift;            // their chunk is 1 << shift pages
+        uint64_t slots;            // partial states per KV head they take
     };
-    const uint64_t whole = makespan();
-    uint64_t best = whole - whole / 20;
-    if (sum / cols >= best) return;   // no split ends before the mean load
-    for (uint32_t r : {n % cols, n % cols + cols / 4}) {
-        if (r >= n) continue;
-        for (uint32_t ch : {16u, 32u, 64u, 128u}) {
-            cost.clear();
-            uint64_t slots_used = 0;
-            for (uint32_t i = 0; i < n; ++i) {
-                const PrefillBlock& b = blk[order[i]];
-                uint64_t p = 0, k = 0;
-                if (i >= n - r)
-                    for (; p + ch <= b.plast; p += ch, ++k) cost.push_back(prefill_cost(ch, b.tiles) + kPrefillSplitCost);
-                cost.push_back(prefill_cost(b.pages - p, b.tiles) + (k ? kPrefillSplitCost : 0));
-                if (k) slots_used += (k + 1) * b.rows;
+    std::vector<Candidate> cand;
+    for (size_t r : {rem, rmax}) {
+        if (r == rem && !cand.empty()) break;   // rmax == rem
+        for (uint32_t shift : {4u, 5u, 6u, 7u}) {
+            uint64_t used = 0;
+            for (size_t i = n - r; i < n; ++i) {
+                const PrefillBlock& b = block(key[i]);
+                const uint64_t k = b.plast >> shift;
+                used += k ? (k + 1) * b.rows : 0;
             }
-            std::sort(cost.begin(), cost.end(), std::greater<uint64_t>());
-            // Merge: its launch (about six page pairs) and reading the states.
             // The workspace stays within what the whole plan asks for (f32
             // states of half as many queries).
-            if (2 * slots_used > queries) continue;
-            const uint64_t e = makespan() + 120 + 8 * slots_used * hkv / slots;
-            if (e < best) {
-                best = e;
-                split = r;
-                chunk = ch;
-            }
+            if (used && 2 * used <= queries) cand.push_back(Candidate{r, shift, used});
         }
     }
+    if (cand.empty()) return {};
+    std::sort(key.begin(), key.end() - rmax, std::greater<uint64_t>());
+    std::vector<uint64_t> whole(n), piece, cost;
+    uint64_t sum = 0;
+    for (size_t i = 0; i < n; ++i) sum += whole[i] = prefill_cost(block(key[i]).pages, block(key[i]).tiles);
+    uint64_t best = prefill_makespan(whole, cols, UINT64_MAX);
+    best -= best / 20;
+    if (sum / cols >= best) return {};   // no split ends before the mean load
+    size_t split = 0;
+    for (const Candidate& c : cand) {
+        piece.clear();
+        uint64_t load = sum;
+        for (size_t i = n - c.r; i < n; ++i) {
+            const PrefillBlock& b = block(key[i]);
+            const uint64_t k = b.plast >> c.shift;
+            piece.insert(piece.end(), k, prefill_cost(uint64_t(1) << c.shift, b.tiles) + kPrefillSplitCost);
+            piece.push_back(prefill_cost(b.pages - (k << c.shift), b.tiles) + (k ? kPrefillSplitCost : 0));
+            load += (k ? (k + 1) * kPrefillSplitCost : 0) + prefill_cost(0, 0) * k;
+        }
+        // Merge: its launch (about six page pairs) and reading the states.
+        const uint64_t merge = 120 + 8 * c.slots * hkv / slots;
+        if (load / cols + merge >= best) continue;
+        std::sort(piece.begin(), piece.end(), std::greater<uint64_t>());
+        cost.resize(n - c.r + piece.size());
+        std::merge(whole.begin(), whole.end() - c.r, piece.begin(), piece.end(), cost.begin(), std::greater<uint64_t>());
+        const uint64_t e = prefill_makespan(cost, cols, best - merge) + merge;
+        if (e < best) {
+            best = e;
+            split = c.r;
+            chunk = 1u << c.shift;
+        }
+    }
+    std::vector<uint32_t> out;
+    for (size_t i = n - split; i < n; ++i) out.push_back(UINT32_MAX - uint32_t(key[i]));
+    return out;
 }
 
 // Prefill items: for each sequence, KV head and block of query tokens
@@ -778,9 +809,11 @@ int build_prefill_plan(const PrefillInput& in, HostPlan& out, std::string& err) 
     };
     std::vector<Piece> pieces;
     // Blocks in (sequence, token) order; of a plan of whole blocks, those of
-    // its tail get a chunk size of their own.
-    std::vector<uint32_t> block_chunk(n_blocks, chunk);
-    if (whole) {
+    // its tail get a chunk size of their own.  Below one round there is no
+    // tail, and beyond eight its idle share is small.
+    std::vector<uint32_t> block_chunk;
+    const uint32_t cols = std::max(1u, in.wg_slots / in.hkv);
+    if (whole && n_blocks > cols && n_blocks / cols < 8 && n_blocks % cols) {
         std::vector<PrefillBlock> blk;
         blk.reserve(n_blocks);
         bool fits = true;
@@ -792,15 +825,13 @@ int build_prefill_plan(const PrefillInput& in, HostPlan& out, std::string& err) 
                                            ((i1 - i0) * r + kTileRows - 1) / kTileRows, i1 - i0});
                 fits = fits && pend <= kPrefillMaxChunk;
             }
-        std::vector<uint32_t> order(blk.size());
-        for (uint32_t i = 0; i < order.size(); ++i) order[i] = i;
-        std::stable_sort(order.begin(), order.end(), [&](uint32_t x, uint32_t y) {
-            return blk[x].pages * (2 + blk[x].tiles) > blk[y].pages * (2 + blk[y].tiles);
-        });
-        uint32_t split = 0, tail_chunk = 0;
-        if (fits) prefill_tail(blk, order, in.wg_slots, in.hkv, nq, split, tail_chunk);
-        for (uint32_t i = 0; i < split; ++i) block_chunk[order[order.size() - 1 - i]] = tail_chunk;
-        out.split_tail = split > 0;
+        uint32_t tail_chunk = 0;
+        if (fits)
+            for (uint32_t i : prefill_tail(blk, cols, in.wg_slots, in.hkv, nq, tail_chunk)) {
+                if (block_chunk.empty()) block_chunk.assign(n_blocks, chunk);
+                block_chunk[i] = tail_chunk;
+            }
+        out.split_tail = !block_chunk.empty();
     }
     size_t block = 0;
     for (uint32_t b = 0; b < B; ++b) {
@@ -811,7 +842,7 @@ int build_prefill_plan(const PrefillInput& in, HostPlan& out, std::string& err) 
             const uint32_t plast = (lmin - 1) / kPageSize;       // a chunk may start at or below this page
             uint32_t p0 = 0;
             while (true) {
-                const uint64_t nx = uint64_t(p0) + block_chunk[block];
+                const uint64_t nx = uint64_t(p0) + (block_chunk.empty() ? chunk : block_chunk[block]);
                 if (nx > plast || nx >= pend) {
                     pieces.push_back(Piece{b, i0, i1, p0, pend});
                     break;
@@ -852,6 +883,7 @@ int build_prefill_plan(const PrefillInput& in, HostPlan& out, std::string& err) 
         ItemLim lim;
     };
     std::vector<Cand> cands;
+    cands.reserve(pieces.size() * in.hkv);
     for (const Piece& pc : pieces) {
         const uint32_t seq_off = uint32_t(out.seqslots.size());
         for (uint32_t i = pc.i0; i < pc.i1; ++i) {
@@ -881,6 +913,9 @@ int build_prefill_plan(const PrefillInput& in, HostPlan& out, std::string& err) 
         out.page_reads += uint64_t(pc.p1 - pc.p0);
     }
     std::stable_sort(cands.begin(), cands.end(), [](const Cand& x, const Cand& y) { return x.cost > y.cost; });
+    out.tasks.reserve(cands.size());
+    out.items.reserve(cands.size());
+    out.item_lim.reserve(cands.size());
     for (const Cand& c : cands) {
         out.tasks.push_back(Task{kTaskGroup, uint32_t(out.items.size()), 1u, 0u});
         out.items.push_back(c.it);
