@@ -179,6 +179,11 @@ __device__ __forceinline__ void row_target(const AttendArgs& a, const Item& it, 
 
 // Group items of the launch: the plan's count, or on the CSR path what the
 // CSR planning kernel of this call wrote (its group items come first).
+// Without CSR (the plan path's kernels) csr_hdr is null.  The tests of it in
+// this and the next two functions, and the item choice by it in the plan
+// path's kernels, stay for the machine code they give those: a 64-leaf bf16
+// tree takes 24.41 us a step with them and 24.52 without, 8 trees of 8 leaves
+// at head_dim 256 31.10 and 31.38.
 template <bool CSR>
 __device__ __forceinline__ uint32_t group_item_count(const AttendArgs& a) {
     return CSR || a.csr_hdr ? __builtin_amdgcn_readfirstlane(a.csr_hdr[4]) : a.n_group_items;
@@ -3656,19 +3661,25 @@ hipError_t launch_merge_d(const MergeArgs& a, uint32_t q_dtype, hipStream_t s) {
     if (rows == 0) return hipSuccess;
     dim3 grid((rows + 3) / 4), block(256);
     // Rows of 17-32 states: the scalar form, one pass of 32, below head_dim
-    // 256.  There its 32 rows of 8 bytes a lane take 144 registers, and the
-    // vector form's one pass is faster (8 trees of 8 leaves, 17-32 states,
-    // 16 / 2 heads, bf16: a step 32.4 -> 30.9 us).  Otherwise the
-    // vector form with loads per pass for the plan's most states per row, so
-    // a row loads no state twice; not known on the host (0, the CSR path):
-    // chosen per row from its own count.
+    // 256.  There its 32 rows of 8 bytes a lane take 286 registers, one wave
+    // a SIMD, and the vector form's one pass is faster (8 trees of 8 leaves,
+    // 17-32 states, 16 / 2 heads, bf16: a step 32.4 -> 30.9 us; f32 states
+    // keep the scalar form's 193 registers).  Otherwise the vector form with
+    // loads per pass for the plan's most states per row, so a row loads no
+    // state twice; not known on the host (0, the CSR path): chosen per row
+    // from its own count.
     const int states = a.max_states > 64 ? 64 : int(a.max_states);
     auto go = [&](auto out_tag) {
         constexpr uint32_t OUT = decltype(out_tag)::value;
         using MS = MergeShape<D, OUT>;
         const int need = (states + MS::SPI - 1) / MS::SPI;
+        if constexpr (D < 256 || OUT == 2) {
+            if (states > 16 && states <= 32) {
+                hipLaunchKernelGGL((merge_kernel<D, OUT, 0>), grid, block, 0, s, a);
+                return;
+            }
+        }
         if (states == 0) hipLaunchKernelGGL((merge_kernel<D, OUT, -1>), grid, block, 0, s, a);
-        else if ((D < 256 || OUT == 2) && states > 16 && states <= 32) hipLaunchKernelGGL((merge_kernel<D, OUT, 0>), grid, block, 0, s, a);
         else if (need <= 1) hipLaunchKernelGGL((merge_kernel<D, OUT, 1>), grid, block, 0, s, a);
         else if (need <= 2 && MS::MAX_NV >= 2) hipLaunchKernelGGL((merge_kernel<D, OUT, (MS::MAX_NV >= 2 ? 2 : 1)>), grid, block, 0, s, a);
         else if (need <= 4 && MS::MAX_NV >= 4) hipLaunchKernelGGL((merge_kernel<D, OUT, (MS::MAX_NV >= 4 ? 4 : 1)>), grid, block, 0, s, a);

@@ -294,7 +294,8 @@ typedef struct dh_plan_stats {
     uint32_t num_items;           /* attention work items                     */
     uint32_t num_tasks;           /* workgroups of the attention launch       */
     uint32_t num_group_items;     /* items whose pages four waves share       */
-    uint32_t num_partials;        /* partial states per q head                */
+    uint32_t num_partials;        /* partial states per q head; of a prefill
+                                     plan with split blocks, theirs only     */
     uint32_t direct;              /* 1: no merge launch (dh_plan_options.direct) */
     uint64_t unique_pages;        /* distinct pages read per step             */
     uint64_t page_reads;          /* pages read per step summed over items of
@@ -338,9 +339,14 @@ dh_status dh_plan_inspect(const dh_attn_config* cfg, uint32_t num_pool_pages,
  * K/V written to pages first); chunked prefill over a cached context is
  * q_len < kv_len.  bf16 / f16 queries (BatchPrefillConfig.dtype,
  * flashinfer/batch_prefill.rs:23), over FP8 / MXFP8 KV at head_dim 128 and
- * 256 as well (codes dequantised to the query's type in the kernel).  chunk_pages: KV pages per work item (0 = chosen from the work:
- * one item per block of queries when those fill the chip, else about 1024
- * items); at most about 2040 whatever is asked (an item's page-id list
+ * 256 as well (codes dequantised to the query's type in the kernel).
+ * chunk_pages: KV pages per work item.  0: chosen from the work.  Where the
+ * blocks of queries fill the chip, one item per (block, KV head), which
+ * writes its rows of out; where that would end in a nearly empty round of
+ * workgroups, the blocks with the least work are split into chunks, and a
+ * second, small launch merges their partial states (dh_decode_stages: stage 1
+ * alone leaves those rows unwritten).  Else chunks for about 1024 items, all
+ * rows merged.  At most about 2040 whatever is asked (an item's page-id list
  * holds 2048 entries), so longer contexts always take several items.
  * Host-side, synchronous. */
 dh_status dh_plan_create_prefill(dh_backend* backend, const dh_attn_config* cfg,

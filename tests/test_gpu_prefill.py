@@ -169,8 +169,10 @@ def test_prefill_items_longer_than_decode_items(backend, chunk):
     (128, 8, 128, _lib.DTYPE_BF16, _lib.KV_MXFP8, [1100], [540], False),
     (64, 8, 256, _lib.DTYPE_F16, _lib.KV_F16, [1500], [521], False),
     (128, 8, 64, _lib.DTYPE_F16, _lib.KV_F16, [1300], [1040], False),
-    (128, 8, 64, _lib.DTYPE_F16, _lib.KV_F16, [1500], [536], True)],
-    ids=["bf16", "f16-fp8", "mxfp8", "d256", "d64", "d64-one-round"])
+    (128, 8, 64, _lib.DTYPE_F16, _lib.KV_F16, [1500], [536], True),
+    (128, 8, 128, _lib.DTYPE_BF16, _lib.KV_FP8_E4M3, [1700, 1300, 1500], [185, 170, 177], True),
+    (128, 8, 128, _lib.DTYPE_BF16, _lib.KV_BF16, [1500, 1500, 1500, 1500], [139, 129, 139, 138], True)],
+    ids=["bf16", "f16-fp8", "mxfp8", "d256", "d64", "d64-one-round", "fp8-three", "bf16-four"])
 def test_prefill_split_tail(backend, case):
     """Plans with a few blocks more than whole rounds of the chip: the tail's
     blocks are split, the others write out themselves.  The workspace stays
