@@ -182,8 +182,8 @@ __device__ __forceinline__ void row_target(const AttendArgs& a, const Item& it, 
 // Without CSR (the plan path's kernels) csr_hdr is null.  The tests of it in
 // this and the next two functions, and the item choice by it in the plan
 // path's kernels, stay for the machine code they give those: a 64-leaf bf16
-// tree takes 24.41 us a step with them and 24.52 without, 8 trees of 8 leaves
-// at head_dim 256 31.10 and 31.38.
+// tree took 24.3-24.4 us a step with them and 24.4-24.6 without, in six
+// builds.
 template <bool CSR>
 __device__ __forceinline__ uint32_t group_item_count(const AttendArgs& a) {
     return CSR || a.csr_hdr ? __builtin_amdgcn_readfirstlane(a.csr_hdr[4]) : a.n_group_items;
