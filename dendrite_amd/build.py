@@ -47,7 +47,7 @@ SANITIZE = ["-Xarch_host", "-fsanitize=address", "-Xarch_host", "-fsanitize=unde
 SAN_BUILD = os.path.join(PKG, "_build_san")
 SAN_LIB = os.path.join(SAN_BUILD, "libdendrite_hip.so")
 
-HIP_SOURCES = ["decode_kernels.hip", "write_kernels.hip"]
+HIP_SOURCES = ["decode_kernels.hip", "csr_kernels.hip", "write_kernels.hip"]
 HOST_SOURCES = ["api.cpp", "planner.cpp", "block_model.cpp"]
 TESTDATA_SOURCES = ["synth.cpp"]
 

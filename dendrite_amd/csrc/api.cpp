@@ -1235,7 +1235,7 @@ dh_status dh_decode_csr(dh_backend* be, const dh_pool* pool, const dh_attn_confi
     // them (kCsrExtraGrid); those past the call's units exit at once.
     const uint64_t waves = slots * per_chunk, units = gcap + (waves + dh::kWaves - 1) / dh::kWaves;
     a.csr_grid = uint32_t(std::min(units, uint64_t(batch) * per_chunk / dh::kWaves + dh::kCsrExtraGrid));
-    e = hipError_t(dh::launch_attend(a, a.csr_grid, c.q_dtype, c.kv_format, c.head_dim, false, stream));
+    e = hipError_t(dh::launch_csr_attend(a, c.q_dtype, c.kv_format, c.head_dim, stream));
     if (e != hipSuccess) return fail(DH_EHIP, "attention launch failed: %s", hipGetErrorString(e));
 
     dh::MergeArgs m{};

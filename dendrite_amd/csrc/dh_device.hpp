@@ -225,7 +225,7 @@ DH_HOST_DEVICE inline uint64_t plane_offset(uint32_t page, uint32_t plane, uint3
 
 }  // namespace dh
 
-// Kernel launchers (defined in decode_kernels.hip and write_kernels.hip).
+// Kernel launchers (defined in decode_kernels.hip, csr_kernels.hip and write_kernels.hip).
 // Return hipError_t as int.
 extern "C++" {
 namespace dh {
@@ -253,6 +253,8 @@ int launch_gather(const uint8_t* kv, const uint32_t* pages, uint32_t n_pages, ui
                   uint32_t hkv, uint32_t head_dim, uint32_t elem_bytes, uint8_t* out,
                   void* stream);
 bool attend_supported(uint32_t q_dtype, uint32_t kv_format, uint32_t head_dim);
+// The attention of a CSR call, on AttendArgs::csr_grid workgroups.
+int launch_csr_attend(const AttendArgs& a, uint32_t q_dtype, uint32_t kv_format, uint32_t head_dim, void* stream);
 int launch_csr_plan(const CsrPlanArgs& p, void* stream);
 int launch_csr_lcp(const int32_t* indptr, const int32_t* indices, uint32_t batch, uint32_t page_limit,
                    uint32_t* lcp, void* stream);
