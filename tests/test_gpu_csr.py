@@ -338,6 +338,44 @@ def test_tables_change_between_calls(backend):
                f"cut {cut}")
 
 
+@pytest.mark.parametrize("fmt", [(_lib.DTYPE_F16, _lib.KV_F16), (_lib.DTYPE_F32, _lib.KV_F32),
+                                 (_lib.DTYPE_BF16, _lib.KV_FP8_E4M3)], ids=["f16", "f32", "fp8"])
+def test_more_wave_items_than_the_grid(backend, fmt):
+    """1 100 sequences of 1-3 pages, 8 KV heads: more than 8 192 wave items,
+    one a (sequence, KV head)."""
+    tables, n = [], 0
+    for b in range(1100):
+        k = 1 + b % 3
+        tables.append(list(range(n, n + k)))
+        n += k
+    run = CsrRun(workloads.custom(tables, 16, 8, 64, fmt[0], fmt[1], n, seed=41), backend)
+    got, st = run.run()
+    assert st == _lib.DH_OK and header(run)[1] > 8192
+    _check(run, got, run.reference(), f"8 800 wave items {fmt}")
+
+
+@pytest.mark.parametrize("fmt", [(_lib.DTYPE_F16, _lib.KV_F16), (_lib.DTYPE_BF16, _lib.KV_FP8_E4M3)],
+                         ids=["f16", "fp8"])
+@pytest.mark.parametrize("d", [64, 128])
+def test_more_group_items_than_the_grid(backend, fmt, d):
+    """102 families of five sequences over 8 shared pages, 32 KV heads (16
+    for FP8 at head_dim 64, whose group items have 64 rows) of 16 query
+    heads: 3 264 group items before the wave items."""
+    hkv = 16 if d == 64 and fmt[1] == _lib.KV_FP8_E4M3 else 32
+    tables, n = [], 0
+    for _ in range(102):
+        shared = list(range(n, n + 8))
+        n += 8
+        for _ in range(5):
+            tables.append(shared + [n])
+            n += 1
+    run = CsrRun(workloads.custom(tables, 16 * hkv, hkv, d, fmt[0], fmt[1], n, seed=43), backend)
+    got, st = run.run()
+    assert st == _lib.DH_OK and header(run)[4] > 2048
+    seqs = list(range(0, 510, 17)) + [508, 509]
+    _check(run, got[seqs], run.reference(seqs=seqs), f"3 264 group items {fmt} d={d}")
+
+
 def attention_grid(run):
     """Workgroups of a call's attention launch (kCsrExtraGrid in
     dh_device.hpp), where the workspace holds more units than that."""
@@ -347,7 +385,7 @@ def attention_grid(run):
 
 @pytest.mark.parametrize("fmt", [(_lib.DTYPE_F16, _lib.KV_F16), (_lib.DTYPE_F32, _lib.KV_F32),
                                  (_lib.DTYPE_BF16, _lib.KV_FP8_E4M3)], ids=["f16", "f32", "fp8"])
-def test_more_wave_items_than_the_grid(backend, fmt):
+def test_second_units_wave_items(backend, fmt):
     """20 sequences of 2 560 table entries over 64 pages, 32 KV heads: ten
     chunks or more a (sequence, KV head), more units than workgroups, so
     workgroups take a second one."""
@@ -366,7 +404,7 @@ def test_more_wave_items_than_the_grid(backend, fmt):
                                  (256, _lib.DTYPE_BF16, _lib.KV_BF16), (256, _lib.DTYPE_F16, _lib.KV_FP8_E4M3)],
                          ids=["d64-f16", "d64-fp8", "d128-bf16", "d128-fp8", "d128-mxfp8", "d128-f16q-mxfp8",
                               "d256-bf16", "d256-f16q-fp8"])
-def test_more_group_items_than_the_grid(backend, fmt):
+def test_second_units_group_items(backend, fmt):
     """100 families of two sequences over 17 shared pages, 32 KV heads of 16
     query heads: 3 200 group items for 2 624 workgroups, so some run a second
     group item, and others a wave item after one, in the same LDS."""
